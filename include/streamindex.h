@@ -74,6 +74,25 @@ int si_indexer_topk(const void* q, const int64_t* q_strides, const void* k_idx, 
                     int64_t top_k, int64_t causal_ratio, int64_t* out_idx, float* out_scores, void* stream);
 
 /*
+ * si_indexer_topk with an optional device scratch of scratch_bytes bytes
+ * (16-byte aligned, free again once the stream has run the call).  Calls with
+ * few query rows and many keys (a decode step, a chunk of a long prompt) then
+ * split the keys over the whole GPU: scores go to the scratch and a second
+ * kernel selects.  Same results, bit for bit.  si_indexer_topk_scratch_bytes
+ * says how much such a call needs; it returns 0 for calls that take none, and
+ * with a scratch that is NULL or smaller the call runs as si_indexer_topk.
+ * No counterpart in the reference (its driver always materialises a score
+ * tile, chunked_indexer.py:92-118).
+ */
+int64_t si_indexer_topk_scratch_bytes(int64_t B, int64_t S, int64_t T, int64_t H, int64_t D, int64_t top_k,
+                                      int64_t causal_ratio);
+int si_indexer_topk_scratch(const void* q, const int64_t* q_strides, const void* k_idx, const int64_t* k_strides,
+                            const void* weights, int w_dtype, const int64_t* w_strides, const uint8_t* mask,
+                            const int64_t* mask_strides, int64_t B, int64_t S, int64_t T, int64_t H, int64_t D,
+                            int64_t top_k, int64_t causal_ratio, int64_t* out_idx, float* out_scores, void* scratch,
+                            int64_t scratch_bytes, void* stream);
+
+/*
  * Which top-k kernel si_indexer_topk and si_csa_indexer_topk launch
  * (process-wide; returns the previous setting).  No counterpart in the
  * reference: a tuning and test knob.  SI_TOPK_KERNEL_AUTO (default) runs

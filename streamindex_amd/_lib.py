@@ -38,6 +38,9 @@ SIGNATURES = {
     "si_indexer_topk_plan": (_I32, [_I64, _I64, _I64, _I64, _I64, _I64, _P, _P]),
     "si_indexer_topk": (_I32, [_P, _I64P, _P, _I64P, _P, _I32, _I64P, _P, _I64P,
                                _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P]),
+    "si_indexer_topk_scratch_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64, _I64, _I64]),
+    "si_indexer_topk_scratch": (_I32, [_P, _I64P, _P, _I64P, _P, _I32, _I64P, _P, _I64P,
+                                       _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _P]),
     "si_indexer_score": (_I32, [_P, _I64P, _P, _I64P, _P, _I32, _I64P,
                                 _I64, _I64, _I64, _I64, _I64, _P, _I64P, _P]),
     "si_csa_indexer_topk": (_I32, [_P, _I64P, _P, _I64P, _P, _I32, _I64P, _I64, _I64, _I64, _I64, _I64,

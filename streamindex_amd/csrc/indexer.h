@@ -33,6 +33,7 @@ struct IndexerArgs {
   float* scores;        // score kernel: [B,S,T]
   int64_t ssb, sss, sst;
   int accumulate;       // score kernel: add to the scores already stored (a later head group)
+  int score_tiles;      // score kernel: key tiles per workgroup (set by launch_score)
 };
 
 // Selection-buffer capacities the top-k kernel is instantiated for: 256,
@@ -78,6 +79,16 @@ inline bool topk_wide_preferred(const IndexerArgs& a) {
 
 template <int HB, int D>
 int launch_score(const IndexerArgs& a, hipStream_t st);
+
+// Scores of calls with fewer than 8 query rows per batch (contiguous key
+// columns, no accumulation): indexer_score_direct_kernel, indexer_topk_few.h.
+template <int HB, int D>
+int launch_score_direct(const IndexerArgs& a, hipStream_t st);
+
+// Second pass of the few-row top-k: the exact top-k of `rows` score rows (or,
+// with `keys`, of rows of selection keys), see indexer_topk_few.h.
+struct FewSelectArgs;
+int launch_few_select(const FewSelectArgs& f, int64_t rows, bool keys, hipStream_t st);
 
 // Head-split top-k kernel (indexer_topk_split.h): HS waves per query row,
 // HBH 32-head blocks per wave, selection capacity C.

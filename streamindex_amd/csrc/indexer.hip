@@ -2,12 +2,26 @@
 // Kernels: indexer_kernels.h (instantiated per head dim in indexer_inst_d*.hip).
 #include <string>
 
-#include "indexer.h"
-#include "si_status.h"
+#include "indexer_topk_few.h"
 
 namespace si {
 
 int g_topk_kernel_mode = 0;
+
+// When the few-row top-k runs (few_plan): at most kFewMaxGroups four-row
+// groups (one per CU), rows of at least kFewMinKeys keys, no causal ratio (its
+// rows are short while they are few), and a scratch within kFewMaxScratch.
+// us a call, one-wave-per-row kernel against this one, H = 64, D = 128,
+// k = 512 (22 us is the host's share of a call):
+//   rows x keys   1 x 1,024   30 -> 22     4 x 16,384 (four batches)  203 -> 23
+//   1 x 65,536   754 -> 27    1 x 262,144  2,910 -> 35
+//   256 x 8,192  146 -> 45    512 x 32,768  460 -> 263
+//   1,024 x 2,048   62 -> 55    1,024 x 32,000   511 -> 469   256 batches x 4,096  80 -> 54
+// and past the line 1,536 x 2,048  79 -> 85, 2,048 x 32,000  818 -> 916: there
+// the one-wave-per-row kernel fills the chip and saves the scores' round trip.
+constexpr int64_t kFewMaxGroups = 256;
+constexpr int kFewMinKeys = 1024;
+constexpr int64_t kFewMaxScratch = int64_t(256) << 20;
 
 // Kernel and selection capacity for a top-k shape.  A compaction keeps
 // between top_k and C - 192 keys; the capacity leaves room for several
@@ -124,6 +138,89 @@ static int dispatch_topk(const IndexerArgs& a, int D, hipStream_t st) {
   return set_error(SI_ERR_UNSUPPORTED, "no top-k kernel for this plan");
 }
 
+// ---------------------------------------------------------------------------
+// Few query rows, many keys: scores to a scratch, then a workgroup per row
+// selects (indexer_topk_few.h).
+// ---------------------------------------------------------------------------
+struct FewPlan {
+  bool use;
+  int64_t sstride;  // floats per scratch score row
+  int64_t segs;     // selection segments per row
+  int64_t bytes;    // scratch: scores, then the segments' keys
+};
+
+static FewPlan few_plan(const IndexerArgs& a, int D) {
+  FewPlan f{};
+  TopkPlan p{};
+  if (g_topk_kernel_mode != 0 || a.ratio > 0 || a.T < kFewMinKeys) return f;
+  if (static_cast<int64_t>(a.B) * ((a.S + 3) / 4) > kFewMaxGroups) return f;
+  if (plan_topk(a, D, &p) != SI_OK || p.kernel == TOPK_SPLIT) return f;
+  const int64_t rows = static_cast<int64_t>(a.B) * a.S;
+  f.sstride = (static_cast<int64_t>(a.T) + 63) / 64 * 64;
+  f.segs = (static_cast<int64_t>(a.T) + kFewSeg - 1) / kFewSeg;
+  if (f.segs > 1 && f.segs * a.top_k > kFewMergeMax) return f;
+  f.bytes = rows * f.sstride * 4 + (f.segs > 1 ? rows * f.segs * a.top_k * 8 : 0);
+  if (f.bytes > kFewMaxScratch) return f;
+  f.use = true;
+  return f;
+}
+
+template <int HB, int D>
+static int launch_few_score(const IndexerArgs& a, hipStream_t st) {
+  return a.S < 8 ? launch_score_direct<HB, D>(a, st) : launch_score<HB, D>(a, st);
+}
+
+static int run_few(const IndexerArgs& a0, const FewPlan& f, int D, void* scratch, hipStream_t st) {
+  IndexerArgs a = a0;
+  a.scores = static_cast<float*>(scratch);
+  a.ssb = a.S * f.sstride;
+  a.sss = f.sstride;
+  a.sst = 1;
+  a.accumulate = 0;
+  const int64_t rows = static_cast<int64_t>(a.B) * a.S;
+  const int HB = (a.H + 31) / 32;
+  int rc = -1;
+#define SI_CASE(hb, d) \
+  if (HB == hb && D == d) rc = launch_few_score<hb, d>(a, st);
+  SI_CASE(1, 32)
+  SI_CASE(1, 64)
+  SI_CASE(1, 128)
+  SI_CASE(1, 256)
+  SI_CASE(2, 32)
+  SI_CASE(2, 64)
+  SI_CASE(2, 128)
+  SI_CASE(2, 256)
+  SI_CASE(3, 32)
+  SI_CASE(3, 64)
+  SI_CASE(3, 128)
+  SI_CASE(4, 32)
+  SI_CASE(4, 64)
+  SI_CASE(4, 128)
+#undef SI_CASE
+  if (rc < 0) return set_error(SI_ERR_UNSUPPORTED, "no score kernel for this shape");
+  if (rc) return rc;
+  FewSelectArgs s{};
+  s.scores = a.scores;
+  s.sstride = f.sstride;
+  s.n = a.T;
+  s.S = a.S;
+  s.top_k = a.top_k;
+  s.mask = a.mask;
+  s.msb = a.msb;
+  s.mss = a.mss;
+  s.mst = a.mst;
+  s.out_idx = a.out_idx;
+  s.out_scores = a.out_scores;
+  if (f.segs > 1) s.seg_keys = reinterpret_cast<uint64_t*>(a.scores + rows * f.sstride);
+  rc = launch_few_select(s, rows, false, st);
+  if (rc || f.segs == 1) return rc;
+  s.keys = s.seg_keys;
+  s.n = static_cast<int>(f.segs * a.top_k);
+  s.mask = nullptr;
+  s.seg_keys = nullptr;
+  return launch_few_select(s, rows, true, st);
+}
+
 // Materialised scores.  A launch covers up to four 32-head blocks (two at
 // D = 256); wider rows run one launch per head group, each after the first
 // adding its part to the scores already written (the same stream orders them).
@@ -223,11 +320,37 @@ extern "C" int si_indexer_topk_plan(int64_t S, int64_t T, int64_t H, int64_t D, 
   return SI_OK;
 }
 
+extern "C" int64_t si_indexer_topk_scratch_bytes(int64_t B, int64_t S, int64_t T, int64_t H, int64_t D,
+                                                 int64_t top_k, int64_t causal_ratio) {
+  const int64_t lim = 0x7fffffff;
+  if (B <= 0 || S <= 0 || T <= 0 || H <= 0 || top_k <= 0 || B > lim || S > lim || T > lim || H > lim || top_k > lim)
+    return 0;
+  IndexerArgs a{};
+  a.B = static_cast<int>(B);
+  a.S = static_cast<int>(S);
+  a.T = static_cast<int>(T);
+  a.H = static_cast<int>(H);
+  a.top_k = static_cast<int>(top_k);
+  a.ratio = causal_ratio > 0 ? 1 : 0;
+  const FewPlan f = few_plan(a, static_cast<int>(D));
+  return f.use ? f.bytes : 0;
+}
+
 extern "C" int si_indexer_topk(const void* q, const int64_t* q_strides, const void* k_idx,
                                const int64_t* k_strides, const void* weights, int w_dtype,
                                const int64_t* w_strides, const uint8_t* mask, const int64_t* mask_strides,
                                int64_t B, int64_t S, int64_t T, int64_t H, int64_t D, int64_t top_k,
                                int64_t causal_ratio, int64_t* out_idx, float* out_scores, void* stream) {
+  return si_indexer_topk_scratch(q, q_strides, k_idx, k_strides, weights, w_dtype, w_strides, mask, mask_strides, B, S,
+                                 T, H, D, top_k, causal_ratio, out_idx, out_scores, nullptr, 0, stream);
+}
+
+extern "C" int si_indexer_topk_scratch(const void* q, const int64_t* q_strides, const void* k_idx,
+                                       const int64_t* k_strides, const void* weights, int w_dtype,
+                                       const int64_t* w_strides, const uint8_t* mask, const int64_t* mask_strides,
+                                       int64_t B, int64_t S, int64_t T, int64_t H, int64_t D, int64_t top_k,
+                                       int64_t causal_ratio, int64_t* out_idx, float* out_scores, void* scratch,
+                                       int64_t scratch_bytes, void* stream) {
   IndexerArgs a{};
   int rc = fill_common(a, q, q_strides, k_idx, k_strides, weights, w_dtype, w_strides, B, S, T, H, D);
   if (rc) return rc;
@@ -244,6 +367,12 @@ extern "C" int si_indexer_topk(const void* q, const int64_t* q_strides, const vo
   a.out_idx = out_idx;
   a.out_scores = out_scores;
   if (a.B == 0 || a.S == 0) return SI_OK;
+  if (scratch) {
+    if (reinterpret_cast<uintptr_t>(scratch) & 15) return set_error(SI_ERR_INVALID, "scratch must be 16-byte aligned");
+    const FewPlan f = few_plan(a, static_cast<int>(D));
+    if (f.use && scratch_bytes >= f.bytes)
+      return run_few(a, f, static_cast<int>(D), scratch, static_cast<hipStream_t>(stream));
+  }
   return dispatch_topk(a, static_cast<int>(D), static_cast<hipStream_t>(stream));
 }
 

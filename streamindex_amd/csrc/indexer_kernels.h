@@ -537,6 +537,7 @@ void indexer_topk_kernel(IndexerArgs a) {
 
 // ---------------------------------------------------------------------------
 // Materialised score matrix [B, S, T] fp32 (no mask, as the reference kernel).
+// The grid's y axis splits the keys into chunks of score_tiles tiles.
 // ---------------------------------------------------------------------------
 template <int HB, int D, int NW, int TILE_N>
 __global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a) {
@@ -560,14 +561,16 @@ __global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a
 
   KTileLoader<D, TILE_N, NT> ld;
   ld.init(a.kst);
-  const int ntiles = (a.T + TILE_N - 1) / TILE_N;
-  if (ntiles > 0) ld.issue(kb, a.kst, 0, a.T, lds);
+  const int it0 = static_cast<int>(blockIdx.y) * a.score_tiles;
+  const int left = (a.T + TILE_N - 1) / TILE_N - it0;
+  const int ntiles = it0 + (left < a.score_tiles ? left : a.score_tiles);
+  if (it0 < ntiles) ld.issue(kb, a.kst, it0 * TILE_N, a.T, lds);
   tile_barrier();
   static_assert(NB % 2 == 0, "32-key blocks are stored in pairs");
-  for (int it = 0; it < ntiles; ++it) {
+  for (int it = it0; it < ntiles; ++it) {
     const bool more = it + 1 < ntiles;
-    if (more) ld.issue(kb, a.kst, (it + 1) * TILE_N, a.T, lds + ((it + 1) & 1) * TILE_BYTES);
-    const char* tile = lds + (it & 1) * TILE_BYTES;
+    if (more) ld.issue(kb, a.kst, (it + 1) * TILE_N, a.T, lds + ((it + 1 - it0) & 1) * TILE_BYTES);
+    const char* tile = lds + ((it - it0) & 1) * TILE_BYTES;
     const int tbase = it * TILE_N;
     // Full tiles of a row that overwrites its scores issue exactly NB / 2
     // stores after the copy of tile it+1, so the wait before the barrier

@@ -121,6 +121,20 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
   return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x)));
 }
 
+// Wave-wide sum of an unsigned value, returned uniformly (the steps of
+// wave_max_u32).
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {
+  x += static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xf, 0xf, false));
+  x += static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x4E, 0xf, 0xf, false));
+  x += static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x141, 0xf, 0xf, false));
+  x += static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x140, 0xf, 0xf, false));
+  const auto r16 = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  x = static_cast<uint32_t>(r16[0]) + static_cast<uint32_t>(r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  x = static_cast<uint32_t>(r32[0]) + static_cast<uint32_t>(r32[1]);
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x)));
+}
+
 // Number of set bits of `m` in lanes strictly below this lane.
 __device__ __forceinline__ int lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
