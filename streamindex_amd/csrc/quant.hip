@@ -17,7 +17,10 @@
 // reads: fp8 e4m3 values with one fp32 scale per block, and fp4 e2m1 values
 // packed two per byte (element 2i in the low nibble) with power-of-two
 // (UE8M0) scales.  All are bandwidth-bound: one thread handles 8 elements, a
-// block of `bs` elements is reduced across bs/8 adjacent lanes.
+// block of `bs` elements is reduced across bs/8 adjacent lanes.  (With 8
+// two-byte loads a thread and a 64-bit division to find its block, packing
+// 134M bf16 values to fp4 took 125 us; 64 us, the rate
+// of a copy, with 16-byte loads, shifts and the conversion instruction.)
 #include <hip/hip_fp16.h>
 
 #include <string>
@@ -65,6 +68,47 @@ struct Elt<2> {
     static_cast<__half*>(p)[i] = __float2half_rn(x);
   }
 };
+
+// N consecutive elements as fp32 (N = 1, or a 16-byte vector).
+template <int DT, int N>
+__device__ __forceinline__ void load_vec(const void* p, int64_t i, float (&v)[N]) {
+  if constexpr (N == 1) {
+    v[0] = Elt<DT>::load(p, i);
+  } else if constexpr (DT == 0) {
+    static_assert(N == 4, "16 bytes");
+    const f32x4 w = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = w[e];
+  } else {
+    static_assert(N == 8, "16 bytes");
+    const u32x4 w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p) + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint16_t h = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
+      if constexpr (DT == 1) v[e] = __uint_as_float(static_cast<uint32_t>(h) << 16);
+      else v[e] = __half2float(__ushort_as_half(h));
+    }
+  }
+}
+template <int DT, int N>
+__device__ __forceinline__ void store_vec(void* p, int64_t i, const float (&v)[N]) {
+  if constexpr (N == 1) {
+    Elt<DT>::store(p, i, v[0]);
+  } else if constexpr (DT == 0) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(p) + i) = f32x4{v[0], v[1], v[2], v[3]};
+  } else {
+    u32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (DT == 1)
+        w[e] = (__float_as_uint(bf16_round(v[2 * e])) >> 16) | (__float_as_uint(bf16_round(v[2 * e + 1])) & 0xffff0000u);
+      else
+        w[e] = static_cast<uint32_t>(__half_as_ushort(__float2half_rn(v[2 * e]))) |
+               (static_cast<uint32_t>(__half_as_ushort(__float2half_rn(v[2 * e + 1]))) << 16);
+    }
+    *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(p) + i) = w;
+  }
+}
 
 // Nearest fp8 e4m3 (OCP "fn": bias 7, no infinities, max 448) value to x,
 // ties to even; |x| <= 448 here (callers clamp).  Returns the value as float.
@@ -121,18 +165,33 @@ struct QuantArgs {
   float* scale;     // pack: one scale per block
   int64_t nblocks;
   int bs;           // block size (multiple of 8, bs / 8 a power of two <= 64)
+  int lg;           // log2(bs / 8): the lanes that share a block
+  int vec;          // x is 16-byte aligned
   int mode;         // pack: 0 = fp32 scale (amax / max), 1 = power-of-two (UE8M0) scale
 };
 
 template <int DT>
-__device__ __forceinline__ float block_amax(const QuantArgs& q, int64_t blk, int sub, int g, float (&v)[8]) {
-  const int64_t base = blk * q.bs + sub * 8;
+__device__ __forceinline__ float block_amax(const QuantArgs& q, int64_t base, int g, float (&v)[8]) {
   float m = 0.f;
+  if (q.vec) {
+    if constexpr (DT == 0) {
+      float a[4], b[4];
+      load_vec<0, 4>(q.x, base, a);
+      load_vec<0, 4>(q.x, base + 4, b);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    v[e] = Elt<DT>::load(q.x, base + e);
-    m = __builtin_fmaxf(m, __builtin_fabsf(v[e]));
+      for (int e = 0; e < 4; ++e) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+      }
+    } else {
+      load_vec<DT, 8>(q.x, base, v);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = Elt<DT>::load(q.x, base + e);
   }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = __builtin_fmaxf(m, __builtin_fabsf(v[e]));
   for (int w = 1; w < g; w <<= 1) m = __builtin_fmaxf(m, __shfl_xor(m, w, 64));
   return m;
 }
@@ -142,16 +201,15 @@ __device__ __forceinline__ float block_amax(const QuantArgs& q, int64_t blk, int
 // the dtype as torch does).
 template <int DT>
 __global__ __launch_bounds__(256) void fp8_simulate_kernel(QuantArgs q) {
-  const int g = q.bs / 8;  // lanes per block
+  const int g = 1 << q.lg;  // lanes per block
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t blk = t / g;
-  const int sub = static_cast<int>(t % g);
+  const int64_t blk = t >> q.lg;
   if (blk >= q.nblocks) return;  // whole lane groups leave together (g divides 64)
   float v[8];
-  float amax = block_amax<DT>(q, blk, sub, g, v);
+  float amax = block_amax<DT>(q, t * 8, g, v);
   amax = Elt<DT>::round(__builtin_fmaxf(amax, 1e-4f));
   const float scale = Elt<DT>::round(amax / 448.f);
-  const int64_t base = blk * q.bs + sub * 8;
+  const int64_t base = t * 8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float y = Elt<DT>::round(v[e] / scale);
@@ -165,16 +223,15 @@ __global__ __launch_bounds__(256) void fp8_simulate_kernel(QuantArgs q) {
 // dtype) -> grid value * scale.
 template <int DT>
 __global__ __launch_bounds__(256) void fp4_simulate_kernel(QuantArgs q) {
-  const int g = q.bs / 8;
+  const int g = 1 << q.lg;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t blk = t / g;
-  const int sub = static_cast<int>(t % g);
+  const int64_t blk = t >> q.lg;
   if (blk >= q.nblocks) return;
   float v[8];
-  float amax = block_amax<DT>(q, blk, sub, g, v);
+  float amax = block_amax<DT>(q, t * 8, g, v);
   amax = Elt<DT>::round(__builtin_fmaxf(amax, 6.f * 0x1p-126f));
   const float scale = Elt<DT>::round(amax / 6.f);
-  const int64_t base = blk * q.bs + sub * 8;
+  const int64_t base = t * 8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float y = Elt<DT>::round(v[e] / scale);
@@ -204,16 +261,15 @@ __device__ __forceinline__ float pow2_ceil(float x) {  // smallest 2^k >= x (x >
 // or its power-of-two ceiling (mode 1); value = e4m3(clamp(x / scale, +-448)).
 template <int DT>
 __global__ __launch_bounds__(256) void fp8_pack_kernel(QuantArgs q) {
-  const int g = q.bs / 8;
+  const int g = 1 << q.lg;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t blk = t / g;
-  const int sub = static_cast<int>(t % g);
+  const int64_t blk = t >> q.lg;
   if (blk >= q.nblocks) return;
   float v[8];
-  const float amax = __builtin_fmaxf(block_amax<DT>(q, blk, sub, g, v), 1e-4f);
+  const float amax = __builtin_fmaxf(block_amax<DT>(q, t * 8, g, v), 1e-4f);
   float scale = amax / 448.f;
   if (q.mode == 1) scale = pow2_ceil(scale);
-  if (sub == 0) q.scale[blk] = scale;
+  if ((t & (g - 1)) == 0) q.scale[blk] = scale;
   uint32_t w[2] = {0u, 0u};
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -221,26 +277,42 @@ __global__ __launch_bounds__(256) void fp8_pack_kernel(QuantArgs q) {
     y = __builtin_fminf(__builtin_fmaxf(y, -448.f), 448.f);
     w[e >> 2] |= static_cast<uint32_t>(e4m3_bits(e4m3_round(y))) << (8 * (e & 3));
   }
-  *reinterpret_cast<uint2*>(static_cast<uint8_t*>(q.y) + blk * q.bs + sub * 8) = uint2{w[0], w[1]};
+  *reinterpret_cast<uint2*>(static_cast<uint8_t*>(q.y) + t * 8) = uint2{w[0], w[1]};
 }
 
 // fp4 e2m1 packed two per byte (element 2i low nibble) + power-of-two scale
 // per block: scale = 2^ceil(log2(max(amax, 6 * 2^-126) / 6)), so |x / scale| <= 6.
 template <int DT>
 __global__ __launch_bounds__(256) void fp4_pack_kernel(QuantArgs q) {
-  const int g = q.bs / 8;
+  const int g = 1 << q.lg;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t blk = t / g;
-  const int sub = static_cast<int>(t % g);
+  const int64_t blk = t >> q.lg;
   if (blk >= q.nblocks) return;
   float v[8];
-  const float amax = __builtin_fmaxf(block_amax<DT>(q, blk, sub, g, v), 6.f * 0x1p-126f);
+  const float amax = __builtin_fmaxf(block_amax<DT>(q, t * 8, g, v), 6.f * 0x1p-126f);
   const float scale = pow2_ceil(amax / 6.f);
-  if (sub == 0) q.scale[blk] = scale;
+  if ((t & (g - 1)) == 0) q.scale[blk] = scale;
   uint32_t w = 0u;
+  const float inv = 1.f / scale;  // exact, as is the product: scale is a normal power of two up to 2^126
 #pragma unroll
-  for (int e = 0; e < 8; ++e) w |= e2m1_code(v[e] / scale) << (4 * e);
-  *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(q.y) + (blk * q.bs + sub * 8) / 2) = w;
+  for (int e = 0; e < 8; ++e) v[e] *= inv;
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) nan |= __builtin_isunordered(v[e], v[e + 1]);
+  if (__builtin_amdgcn_ballot_w64(nan || !(amax < __builtin_inff())) == 0) {
+    // The conversion instruction rounds as e2m1_code does but keeps the sign of
+    // a value that rounds to zero (e2m1_code: 130 instructions for the 8).
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[0], v[1], 1.0f, 0);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[2], v[3], 1.0f, 1);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[4], v[5], 1.0f, 2);
+    w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[6], v[7], 1.0f, 3);
+    const uint32_t nonzero = (w | (w >> 1) | (w >> 2)) & 0x11111111u;
+    w &= 0x77777777u | (nonzero << 3);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w |= e2m1_code(v[e]) << (4 * e);
+  }
+  *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(q.y) + t * 4) = w;
 }
 
 // ---- token compressor / softmax-gated pool ----------------------------------
@@ -256,38 +328,129 @@ struct PoolArgs {
   int overlap;
 };
 
-// One thread per (batch, compressed entry, channel).  Overlap (CSA, eq. 11-12):
-// softmax over the 2m scores [z_a + b_a of block i ; z_b + b_b of block i-1]
-// (block 0: the b half is -inf / 0); no overlap (HCA, eq. 22-23): softmax over
-// the m scores of block i.  fp32 arithmetic, output rounded to the dtype.
-template <int DT>
+// Overlap (CSA, eq. 11-12): softmax over the 2m scores [z_a + b_a of block i ;
+// z_b + b_b of block i-1] (block 0: the b half is -inf / 0); no overlap (HCA,
+// eq. 22-23): softmax over the m scores of block i.  fp32 arithmetic, output
+// rounded to the dtype.
+//
+// One item per (batch, compressed entry, N channels); R threads of a workgroup
+// share an item, each taking every R-th chunk of U rows, and meet in LDS.
+// Bound: HBM.  Every score and content row is read once, 16 bytes a lane
+// (N = 8, fp32: 4), U scores and U contents in flight per thread, with the
+// running maximum moved once a chunk (an entry of up to U rows never rescales).
+// R = 8 where entries are long and few (m = 128), so that enough loads are in
+// flight.  N = 1 serves the channel counts and addresses that are not whole
+// 16-byte vectors.
+template <int DT, int N, int R>
 __global__ __launch_bounds__(256) void token_compress_kernel(PoolArgs p) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t total = p.B * p.nblk * p.C;
-  if (t >= total) return;
-  const int64_t c = t % p.C;
-  const int64_t i = (t / p.C) % p.nblk;
-  const int64_t b = t / (p.C * p.nblk);
-  const int64_t row0 = (b * p.S + i * p.m) * p.C + c;
-  float mx = -__builtin_inff();
-  for (int64_t j = 0; j < p.m; ++j) mx = __builtin_fmaxf(mx, Elt<DT>::load(p.za, row0 + j * p.C) + p.ba[j * p.C + c]);
-  const bool has_b = p.overlap && i > 0;
-  const int64_t rowb = row0 - p.m * p.C;  // block i-1
-  if (has_b)
-    for (int64_t j = 0; j < p.m; ++j) mx = __builtin_fmaxf(mx, Elt<DT>::load(p.zb, rowb + j * p.C) + p.bb[j * p.C + c]);
-  float den = 0.f, num = 0.f;
-  for (int64_t j = 0; j < p.m; ++j) {
-    const float w = __expf(Elt<DT>::load(p.za, row0 + j * p.C) + p.ba[j * p.C + c] - mx);
-    den += w;
-    num += w * Elt<DT>::load(p.ca, row0 + j * p.C);
+  constexpr int U = 8;
+  constexpr int ITEMS = 256 / R;
+  const int local = static_cast<int>(threadIdx.x) % ITEMS;
+  const int part = static_cast<int>(threadIdx.x) / ITEMS;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * ITEMS + local;
+  const int64_t cv = p.C / N;
+  const bool live = item < p.B * p.nblk * cv;
+  if (R == 1 && !live) return;
+  const int64_t at = live ? item : 0;
+  int64_t c, i, b;
+  if (p.B * p.nblk * cv <= 0x7fffffff) {  // (32-bit divisions where they do)
+    const uint32_t x = static_cast<uint32_t>(at), y = x / static_cast<uint32_t>(cv);
+    c = static_cast<int64_t>(x % static_cast<uint32_t>(cv)) * N;
+    i = y % static_cast<uint32_t>(p.nblk);
+    b = y / static_cast<uint32_t>(p.nblk);
+  } else {
+    c = at % cv * N;
+    i = (at / cv) % p.nblk;
+    b = at / (cv * p.nblk);
   }
-  if (has_b)
-    for (int64_t j = 0; j < p.m; ++j) {
-      const float w = __expf(Elt<DT>::load(p.zb, rowb + j * p.C) + p.bb[j * p.C + c] - mx);
-      den += w;
-      num += w * Elt<DT>::load(p.cb, rowb + j * p.C);
+  const int64_t rowa = (b * p.S + i * p.m) * p.C + c;
+  const int64_t rowb = rowa - p.m * p.C;  // block i-1
+  const int64_t rows = p.overlap && i > 0 ? 2 * p.m : p.m;
+  float mx[N], den[N], num[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    mx[e] = -__builtin_inff();
+    den[e] = 0.f;
+    num[e] = 0.f;
+  }
+  for (int64_t j0 = part * U; j0 < rows; j0 += R * U) {
+    float z[U][N], v[U][N];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = j0 + u;
+      if (j < rows) {
+        const bool second = j >= p.m;
+        const int64_t off = second ? rowb + (j - p.m) * p.C : rowa + j * p.C;
+        float bias[N];
+        load_vec<DT, N>(second ? p.zb : p.za, off, z[u]);
+        load_vec<DT, N>(second ? p.cb : p.ca, off, v[u]);
+        const float* bp = second ? p.bb + (j - p.m) * p.C + c : p.ba + j * p.C + c;
+#pragma unroll
+        for (int e = 0; e < N; e += N < 4 ? N : 4) {
+          if constexpr (N == 1) {
+            bias[0] = bp[0];
+          } else {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(bp + e);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bias[e + q] = w[q];
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < N; ++e) z[u][e] += bias[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          z[u][e] = -__builtin_inff();
+          v[u][e] = 0.f;
+        }
+      }
     }
-  Elt<DT>::store(p.out, t, num / den);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      float m = mx[e];
+#pragma unroll
+      for (int u = 0; u < U; ++u) m = __builtin_fmaxf(m, z[u][e]);
+      const float ref = m == -__builtin_inff() ? 0.f : m;  // (every score so far -inf: all weights 0)
+      const float s = __expf(mx[e] - ref);
+      den[e] *= s;
+      num[e] *= s;
+      mx[e] = m;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float w = __expf(z[u][e] - ref);
+        den[e] += w;
+        num[e] += w * v[u][e];
+      }
+    }
+  }
+  if constexpr (R > 1) {
+    __shared__ float part_lds[R][3 * N][ITEMS];
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      part_lds[part][e][local] = mx[e];
+      part_lds[part][N + e][local] = den[e];
+      part_lds[part][2 * N + e][local] = num[e];
+    }
+    __syncthreads();
+    if (part != 0 || !live) return;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      float m = mx[e];
+      for (int q = 1; q < R; ++q) m = __builtin_fmaxf(m, part_lds[q][e][local]);
+      const float ref = m == -__builtin_inff() ? 0.f : m;
+      float d = 0.f, a = 0.f;
+      for (int q = 0; q < R; ++q) {
+        const float s = __expf(part_lds[q][e][local] - ref);
+        d += part_lds[q][N + e][local] * s;
+        a += part_lds[q][2 * N + e][local] * s;
+      }
+      den[e] = d;
+      num[e] = a;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < N; ++e) num[e] = num[e] / den[e];
+  store_vec<DT, N>(p.out, at * N, num);
 }
 
 // softmax_gated_pool over the middle axis of [outer, L, inner] tensors.
@@ -326,7 +489,36 @@ template <int DT> struct Fp8Sim { static constexpr auto fn = fp8_simulate_kernel
 template <int DT> struct Fp4Sim { static constexpr auto fn = fp4_simulate_kernel<DT>; };
 template <int DT> struct Fp8Pack { static constexpr auto fn = fp8_pack_kernel<DT>; };
 template <int DT> struct Fp4Pack { static constexpr auto fn = fp4_pack_kernel<DT>; };
-template <int DT> struct Compress { static constexpr auto fn = token_compress_kernel<DT>; };
+
+template <int DT, int N, int R>
+static int launch_compress_r(const PoolArgs& p, hipStream_t st) {
+  const int64_t items = p.B * p.nblk * (p.C / N);
+  const int64_t blocks = (items + 256 / R - 1) / (256 / R);
+  if (blocks > 0x7fffffffLL) return set_error(SI_ERR_UNSUPPORTED, "tensor too large");
+  if (blocks == 0) return SI_OK;
+  hipLaunchKernelGGL((token_compress_kernel<DT, N, R>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, p);
+  return check_launch("token_compress_kernel");
+}
+template <int DT>
+static int launch_compress(const PoolArgs& p, hipStream_t st) {
+  constexpr int N = DT == 0 ? 4 : 8;
+  const uintptr_t ptrs = reinterpret_cast<uintptr_t>(p.ca) | reinterpret_cast<uintptr_t>(p.za) |
+                         reinterpret_cast<uintptr_t>(p.cb) | reinterpret_cast<uintptr_t>(p.zb) |
+                         reinterpret_cast<uintptr_t>(p.ba) | reinterpret_cast<uintptr_t>(p.bb) |
+                         reinterpret_cast<uintptr_t>(p.out);
+  if (p.C % N || (ptrs & 15)) return launch_compress_r<DT, 1, 1>(p, st);
+  // Long entries: several threads each, so that their rows load in parallel.
+  return p.m >= 32 ? launch_compress_r<DT, N, 8>(p, st) : launch_compress_r<DT, N, 1>(p, st);
+}
+
+static int log2_lanes(int64_t bs) {
+  int lg = 0;
+  while ((8ll << lg) < bs) ++lg;
+  return lg;
+}
+static int aligned16(const void* x) {
+  return (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+}
 
 static int check_block(int64_t n, int64_t bs) {
   if (bs < 8 || bs > 512 || bs % 8 || ((bs / 8) & (bs / 8 - 1)))
@@ -344,7 +536,7 @@ extern "C" int si_quant_simulate(const void* x, void* y, int dtype, int64_t n, i
   int rc = check_block(n, block_size);
   if (rc) return rc;
   if (n > 0 && (!x || !y)) return set_error(SI_ERR_INVALID, "null pointer argument");
-  QuantArgs q{x, y, nullptr, n / block_size, static_cast<int>(block_size), 0};
+  QuantArgs q{x, y, nullptr, n / block_size, static_cast<int>(block_size), log2_lanes(block_size), aligned16(x), 0};
   const int64_t threads = n / 8;
   hipStream_t st = static_cast<hipStream_t>(stream);
   return fp4 ? launch_dt<Fp4Sim>(dtype, threads, q, "fp4_simulate_kernel", st)
@@ -358,7 +550,8 @@ extern "C" int si_quant_pack(const void* x, void* y, float* scale, int dtype, in
   if (n > 0 && (!x || !y || !scale)) return set_error(SI_ERR_INVALID, "null pointer argument");
   if ((reinterpret_cast<uintptr_t>(y) & 7) || (fp4 && (reinterpret_cast<uintptr_t>(y) & 3)))
     return set_error(SI_ERR_INVALID, "output must be 8-byte aligned");
-  QuantArgs q{x, y, scale, n / block_size, static_cast<int>(block_size), pow2_scale ? 1 : 0};
+  QuantArgs q{x, y, scale, n / block_size, static_cast<int>(block_size), log2_lanes(block_size), aligned16(x),
+              pow2_scale ? 1 : 0};
   const int64_t threads = n / 8;
   hipStream_t st = static_cast<hipStream_t>(stream);
   return fp4 ? launch_dt<Fp4Pack>(dtype, threads, q, "fp4_pack_kernel", st)
@@ -373,7 +566,13 @@ extern "C" int si_token_compress(const void* c_a, const void* z_a, const float* 
   if (B * nblk > 0 && (!c_a || !z_a || !b_a || !out || (overlap && (!c_b || !z_b || !b_b))))
     return set_error(SI_ERR_INVALID, "null pointer argument");
   PoolArgs p{c_a, z_a, c_b, z_b, b_a, b_b, out, B, S, C, m, nblk, overlap ? 1 : 0};
-  return launch_dt<Compress>(dtype, B * nblk * C, p, "token_compress_kernel", static_cast<hipStream_t>(stream));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case 0: return launch_compress<0>(p, st);
+    case 1: return launch_compress<1>(p, st);
+    case 2: return launch_compress<2>(p, st);
+    default: return set_error(SI_ERR_UNSUPPORTED, "dtype must be fp32, bf16 or fp16");
+  }
 }
 
 extern "C" int si_gated_pool(const void* kv, const void* score, void* out, int dtype, int64_t outer, int64_t L,

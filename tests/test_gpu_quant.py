@@ -83,3 +83,52 @@ def test_gated_pool(cuda_device):
         w = np.exp(sc - sc.max(dim, keepdims=True))
         ref = (kv * w).sum(dim) / w.sum(dim)
         assert np.abs(got.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dt,tol", [("float32", 1e-5), ("bfloat16", 2e-2), ("float16", 2e-3)])
+@pytest.mark.parametrize("overlap,m,C,shift", [
+    (True, 5, 40, 0),     # 10 rows: two chunks of 8
+    (True, 4, 44, 0),     # 44 channels are whole 16-byte vectors in fp32 only
+    (True, 4, 37, 0),     # scalar kernel
+    (True, 4, 96, 1),     # rows off the 16-byte grid: scalar kernel
+    (False, 31, 64, 0),   # longest entry of one thread
+    (False, 32, 64, 0),   # shortest entry of eight threads
+    (False, 67, 72, 0),   # eight threads, uneven chunks, a partial workgroup
+    (True, 33, 8, 0),
+])
+def test_token_compressor_chunks(cuda_device, dt, tol, overlap, m, C, shift):
+    # a -inf score has weight 0, also in a chunk of its own before the first finite one
+    rng = np.random.default_rng(m + C)
+    B, S = 2, 3 * m + 1
+    arr = [O.round_to(rng.standard_normal((B, S, C)).astype(np.float32), dt) for _ in range(4)]
+    arr[1][:, m:m + 9] = -np.inf if m > 9 else arr[1][:, m:m + 9]
+    ba, bb = rng.standard_normal((m, C)).astype(np.float32), rng.standard_normal((m, C)).astype(np.float32)
+
+    def dev(a):
+        x = torch.from_numpy(a).to(TD[dt])
+        return torch.empty(x.numel() + shift, dtype=x.dtype, device="cuda")[shift:].view(x.shape).copy_(x)
+
+    t = [dev(a) for a in arr]
+    kw = dict(c_b=t[2], z_b=t[3], b_b=torch.from_numpy(bb).cuda()) if overlap else {}
+    got = compressor.token_compressor(t[0], t[1], torch.from_numpy(ba).cuda(), m, overlap=overlap, **kw)
+    ref = O.token_compressor(arr[0], arr[1], ba, m, arr[2], arr[3], bb, overlap)
+    assert np.abs(got.float().cpu().numpy() - ref).max() <= tol * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+def test_fp4_pack_ties_signs_and_shift(cuda_device, dt):
+    # every rounding tie of the grid and both zeros' neighbourhoods, at a
+    # power-of-two scale; off the 16-byte grid too
+    mid = np.array([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0], np.float32)
+    vals = np.concatenate([mid, mid * 1.01, mid * 0.99, [0, 1e-3, 0.5, 1, 1.5, 2, 3, 4, 6]]).astype(np.float32)
+    vals = np.concatenate([vals, -vals, [6, 6, 6, 6]])[:64]
+    x = O.round_to(np.tile(vals, (3, 2)) * np.float32(2.0 ** -7), dt)
+    x[:, ::32] = 6 * 2.0 ** -7
+    for shift in (0, 1):
+        t = torch.empty(x.size + shift, dtype=TD[dt], device="cuda")[shift:].view(x.shape).copy_(torch.from_numpy(x))
+        p, s = quant.fp4_act_quant(t, 32)
+        rv, rs = O.fp4_pack(x, 32)
+        assert np.array_equal(s.cpu().numpy(), rs)
+        assert np.array_equal(O.fp4_unpack(p.cpu().numpy()), rv)
+        b = p.cpu().numpy()
+        assert not np.any((b & 0xF) == 8) and not np.any((b >> 4) == 8)  # zero has one code
