@@ -183,6 +183,25 @@ int si_sparse_attn_fwd_kv2(const void* q, const int64_t* q_strides, const void* 
                            const int64_t* row_len_strides, void* stream);
 
 /*
+ * The forward with everything optional: a second KV tensor (N_kv2 = 0: none;
+ * with one the indices are int32), row lengths (NULL: none), and a device
+ * scratch of scratch_bytes bytes (16-byte aligned, free again once the stream
+ * has run the call).  With a scratch, calls of few query rows (a decode step)
+ * split each row's columns over several workgroups and combine their fp32
+ * partial outputs.  si_sparse_attn_fwd_scratch_bytes says how much such a call
+ * needs, 0 for calls that take none; with a scratch that is NULL or smaller
+ * the call runs unsplit.  No counterpart in the reference.
+ */
+int64_t si_sparse_attn_fwd_scratch_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int64_t K);
+int si_sparse_attn_fwd_scratch(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,
+                               int64_t N_kv, const void* kv2, const int64_t* kv2_strides, int64_t N_kv2,
+                               const float* attn_sink, const void* topk_idxs, int idx_is_i64,
+                               const int64_t* idx_strides, int64_t B, int64_t S, int64_t H, int64_t D, int64_t K,
+                               float softmax_scale, int qkv_dtype, void* o, const int64_t* o_strides, float* lse,
+                               const int64_t* lse_strides, const int32_t* row_len, const int64_t* row_len_strides,
+                               void* scratch, int64_t scratch_bytes, void* stream);
+
+/*
  * Fused indexer top-k that writes CSA attention index rows directly.
  * Replaces flash_sparse/csa.py:149-179 (chunked indexer, window indices,
  * "+S" offset of the compressed picks, int32 concat) and, for the same

@@ -56,6 +56,10 @@ SIGNATURES = {
     "si_sparse_attn_fwd_kv2": (_I32, [_P, _I64P, _P, _I64P, _I64, _P, _I64P, _I64, _P, _P, _I64P,
                                       _I64, _I64, _I64, _I64, _I64, ctypes.c_float, _I32,
                                       _P, _I64P, _P, _I64P, _P, _I64P, _P]),
+    "si_sparse_attn_fwd_scratch_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64]),
+    "si_sparse_attn_fwd_scratch": (_I32, [_P, _I64P, _P, _I64P, _I64, _P, _I64P, _I64, _P, _P, _I32, _I64P,
+                                          _I64, _I64, _I64, _I64, _I64, ctypes.c_float, _I32,
+                                          _P, _I64P, _P, _I64P, _P, _I64P, _P, _I64, _P]),
     "si_indexer_topk_q": (_I32, [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _P, _I32, _I64P, _P, _I64P,
                                  _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "si_csa_indexer_topk_q": (_I32, [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _P, _I32, _I64P,
@@ -133,6 +137,17 @@ def qkv_dtype(t: torch.Tensor) -> int:
 
 def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def scratch(nbytes: int, device: torch.device):
+    """``(tensor or None, bytes)`` of optional scratch from the caching allocator on the current stream; none where memory
+    has run out (the call then takes the path that needs none)."""
+    if nbytes:
+        try:
+            return torch.empty((nbytes,), dtype=torch.uint8, device=device), nbytes
+        except torch.OutOfMemoryError:
+            pass
+    return None, 0
 
 
 def check(rc: int) -> None:

@@ -12,8 +12,9 @@
 // Design (up to 64 heads of one query row at a time per workgroup of 8 waves:
 // four S^T/softmax "producer" waves and four P.V "consumer" waves, one of
 // each per SIMD, so the matrix cores of a SIMD alternate between the two
-// roles; at D >= 512 a workgroup takes 8 consecutive rows one after the other
-// and fetches each next row's first index words during the current row):
+// roles; at D >= 512 a workgroup takes up to 8 consecutive rows one after the
+// other and fetches each next row's first index words during the current row;
+// with few rows several workgroups share one, attn_plan):
 //   * The row's top-k KV rows are gathered 32 at a time straight from L2/HBM
 //     into a 4-slot LDS ring with global_load_lds (no staging registers) by
 //     the producers, three tiles ahead of use; each row is read once per query
@@ -75,6 +76,12 @@ struct SparseAttnArgs {
   const uint16_t* kv2;
   int64_t kv2sb, kv2sn;
   int N1;
+  // Split rows (ATTN_SPLIT): workgroup `split` of a row runs columns
+  // [split * span, (split + 1) * span) and leaves its unnormalised output and
+  // (reference maximum, denominator) for sparse_attn_combine_kernel.
+  int splits, span;
+  float* part_o;       // [B*S, HG, splits, 64, D]
+  float2* part_ml;     // [B*S, HG, splits, 64]
 };
 
 // The reference maximum of a head moves only when a tile's maximum exceeds it
@@ -91,17 +98,12 @@ constexpr float kLazyRescaleF16 = 8.0f;
 // dealt round-robin), one of each per SIMD.
 constexpr int kAttnThreads = 2 * kAttnWaves * 64;
 
-// Query rows per workgroup (ROWS), handled one after the other: while a
-// row's last tiles run, the index wave copies the next row's first index
-// words, so each row after the first starts without waiting for them (half
-// of a row's prologue at D = 576).  Used where one workgroup fills a CU
-// (D >= 512); with several workgroups per CU the others hide the prologue
-// and a shorter grid only costs (measured: -3 % at D = 576, +27 % at D = 64
-// for 8 rows).
-template <int D>
-constexpr int attn_rows_per_workgroup() {
-  return D >= 512 ? 8 : 1;
-}
+// How rows are dealt to workgroups (attn_plan): several rows per workgroup, one
+// after the other (D >= 512; one row below), one row per workgroup, or several
+// workgroups per row.  A template parameter: the other forms' state does not
+// fit the registers of the first.
+enum AttnMode { ATTN_ROWS = 0, ATTN_ROW = 1, ATTN_SPLIT = 2 };
+constexpr int kAttnManyRows = 8;
 
 // Published KV row offsets: 16-byte units from the batch's first KV row
 // (32 bits) with one KV tensor; with two (KV2) signed byte offsets from the
@@ -110,9 +112,10 @@ constexpr int attn_rows_per_workgroup() {
 template <bool KV2>
 using AttnRowOff = std::conditional_t<KV2, int64_t, uint32_t>;
 
-template <int D, bool IDX64, bool F16, bool KV2>
+template <int D, bool IDX64, bool F16, bool KV2, int MODE>
 __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAttnArgs a) {
-  constexpr int kAttnRows = attn_rows_per_workgroup<D>();
+  constexpr int kAttnRows = MODE == ATTN_ROWS && D >= 512 ? kAttnManyRows : 1;
+  constexpr bool SPLIT = MODE == ATTN_SPLIT;
   using SH = AttnShape<D>;
   constexpr int KS = SH::KS;
   constexpr int MBW = SH::MBW;
@@ -139,8 +142,10 @@ __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAtt
   // (XCD-aware block order, xcd_block_order: HCA attention -2.5 %, CSA
   // attention -2 % at S = 64K, config[3]'s scattered picks unchanged)
   const int lb = xcd_block_order();
-  const int sg = lb % nsg;
-  const int rest = lb / nsg;
+  const int split = SPLIT ? lb % a.splits : 0;
+  const int lr = SPLIT ? lb / a.splits : lb;
+  const int sg = lr % nsg;
+  const int rest = lr / nsg;
   const int b = rest % a.B;
   const int hg = rest / a.B;
   const int hbase = hg * 64;
@@ -153,9 +158,14 @@ __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAtt
       const int rl = a.row_len[b * a.rlsb + static_cast<int64_t>(r) * a.rlss];
       kl = rl < 0 ? 0 : (rl < a.K ? rl : a.K);
     }
+    if constexpr (SPLIT) {  // this workgroup's columns
+      kl -= split * a.span;
+      kl = kl < 0 ? 0 : (kl < a.span ? kl : a.span);
+    }
     return kl;
   };
-  const char* idx_base = static_cast<const char*>(a.idx) + b * a.isb * (IDX64 ? 8 : 4);
+  const char* idx_base = static_cast<const char*>(a.idx) +
+                         (b * a.isb + (SPLIT ? static_cast<int64_t>(split) * a.span * a.isk : 0)) * (IDX64 ? 8 : 4);
   bool idx_ready = false;  // (index wave) this row's first index words were copied during the previous row
   for (int jr = 0; jr < kAttnRows; ++jr) {
     const int s = sg * kAttnRows + jr;
@@ -460,6 +470,13 @@ __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAtt
         const SwapPair r32 = permlane32_swap(__float_as_uint(l_tot), __float_as_uint(l_tot));
         l_tot = __uint_as_float(r32.x) + __uint_as_float(r32.y);
       }
+      if constexpr (SPLIT) {
+        if (g == 0) {
+          const int64_t at = ((static_cast<int64_t>(b) * a.S + s) * a.HG + hg) * a.splits + split;
+          a.part_ml[at * 64 + wave * 16 + i16] = float2{m_ref, l_tot};
+        }
+        return;
+      }
       constexpr float kLog2e = 1.4426950408889634f;
       // (the sink is read only now: a load at the top would make the first
       // copies wait for every Q load)
@@ -636,6 +653,22 @@ __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAtt
         }
       }
       __builtin_amdgcn_s_waitcnt(0x7 << 4);  // no gather may still target the ring
+      if constexpr (SPLIT) {
+        // (64 contiguous bytes of a head per four lanes; heads past H are
+        // written too, they have a row of the scratch)
+        const int64_t at = ((static_cast<int64_t>(b) * a.S + s) * a.HG + hg) * a.splits + split;
+        float* po = a.part_o + at * 64 * D;
+  #pragma unroll
+        for (int j = 0; j < MBW; ++j) {
+          const int mbi = j * kAttnWaves + wave;
+          if (SH::MBT % kAttnWaves == 0 || mbi < SH::MBT) {
+  #pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+              *reinterpret_cast<f32x4*>(po + (nb * 16 + i16) * D + mbi * 16 + 4 * g) = oacc[j][nb];
+          }
+        }
+        return;
+      }
       if (idx_wave) idx_ready = ntiles > 0 && np_nx > 0;
       __syncthreads();  // normalisation factors published
       // Normalised O (bf16) staged head-major in LDS: [64 heads][OROW bytes].
@@ -671,23 +704,143 @@ __global__ __launch_bounds__(kAttnThreads) void sparse_attn_fwd_kernel(SparseAtt
   }
 }
 
-template <int D>
-static int launch_attn(const SparseAttnArgs& a, hipStream_t st) {
-  constexpr int R = attn_rows_per_workgroup<D>();
-  const int64_t nblk = static_cast<int64_t>(a.B) * ((a.S + R - 1) / R) * a.HG;
+// Output and lse of split rows: one thread per four dimensions of a head.
+// Bound: the partial outputs, read once (they fit the last-level cache).
+template <bool F16>
+__global__ __launch_bounds__(256) void sparse_attn_combine_kernel(SparseAttnArgs a, int D) {
+  constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+  const int vec = D / 4;
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t head = e / vec;
+  const int d = static_cast<int>(e - head * vec) * 4;
+  const int64_t row = head / a.H;
+  if (row >= static_cast<int64_t>(a.B) * a.S) return;
+  const int h = static_cast<int>(head - row * a.H);
+  const int b = static_cast<int>(row / a.S), s = static_cast<int>(row % a.S);
+  const int64_t at = (row * a.HG + h / 64) * a.splits;
+  const float2* ml = a.part_ml + at * 64 + h % 64;
+  const float sink2 = a.sink[h] * kLog2e;
+  float m = sink2;
+  for (int i = 0; i < a.splits; ++i) m = __builtin_fmaxf(m, ml[i * 64].x);
+  float l = __builtin_amdgcn_exp2f(sink2 - m);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (a split without a valid key holds zeros; 8 splits' loads in flight)
+  const float* po = a.part_o + (at * 64 + h % 64) * D + d;
+  for (int i = 0; i < a.splits; i += 8) {
+    float2 v[8];
+    f32x4 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int j = i + u < a.splits ? i + u : a.splits - 1;
+      v[u] = ml[j * 64];
+      x[u] = *reinterpret_cast<const f32x4*>(po + static_cast<int64_t>(j) * 64 * D);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float w = i + u < a.splits ? __builtin_amdgcn_exp2f(v[u].x - m) : 0.f;
+      l = __builtin_fmaf(v[u].y, w, l);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = __builtin_fmaf(x[u][c], w, acc[c]);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint2 o;
+  o.x = pack2<F16>(acc[0] * inv, acc[1] * inv);
+  o.y = pack2<F16>(acc[2] * inv, acc[3] * inv);
+  *reinterpret_cast<uint2*>(a.o + b * a.osb + static_cast<int64_t>(s) * a.oss + static_cast<int64_t>(h) * a.osh + d) = o;
+  if (d == 0)
+    a.lse[b * a.lsb + static_cast<int64_t>(s) * a.lss + static_cast<int64_t>(h) * a.lsh] =
+        l > 0.f ? (__builtin_amdgcn_logf(l) + m) * kLn2 : -1.0e30f;
+}
+
+// How the rows are dealt to workgroups.
+//
+// Several rows per workgroup: while a row's last tiles run, the index wave
+// copies the next row's first index words, so each row after the first starts
+// without waiting for them (half of a row's prologue at D = 576).  It pays
+// where one workgroup fills a CU (D >= 512; with several workgroups per CU the
+// others hide the prologue and a shorter grid only costs: +27 % at D = 64 for
+// 8 rows); one row per workgroup costs 14 % more a row.  But 8 rows are also
+// the grain of the grid, so whichever form's busiest CU ends first.  us a call
+// at H = 64, D = 576, K = 512, 8 rows against the choice: S = 300 182 -> 56,
+// S = 1,024 193 -> 131, S = 1,500 213 -> 182, S = 2,048 234 -> 235 (8 rows),
+// S = 2,200 389 -> 250, S = 3,000 393 -> 321, S = 5,000 588 -> 524.
+//
+// Splits: with fewer rows than CUs a row is one workgroup's chain of K / 32
+// tiles while other CUs idle; the second launch and the fp32 partial outputs
+// take back 7 us and 0.6 us a MB, so rows split where that saves a quarter of
+// the estimate: 1 row x K = 2,048 78 -> 27 us, 16 x 2,048 78 -> 31, 16 x 1,024
+// 44 -> 28, 64 x 2,048 79 -> 47; 16 x 512 (25 us) stays whole.
+struct AttnPlan {
+  int mode, splits, span;
+  int64_t bytes;  // scratch of the split rows
+};
+static AttnPlan attn_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t K) {
+  AttnPlan p{ATTN_ROWS, 1, 0, 0};
+  const int64_t hg = (H + 63) / 64;
+  const int64_t units = B * S * hg;
+  if (D >= 512) {
+    constexpr int64_t R = kAttnManyRows;
+    const int64_t blocks = B * ((S + R - 1) / R) * hg;
+    const int64_t full = blocks / 256, left = units - full * 256 * R;
+    const int64_t many = full * R + (left < 0 ? 0 : left < R ? left : R);  // rows of the busiest CU
+    const int64_t one = (units + 255) / 256;
+    if (static_cast<double>(one) * 1.14 < static_cast<double>(many)) p.mode = ATTN_ROW;
+  }
+  const int64_t tiles = (K + kAttnTK - 1) / kAttnTK;
+  if (units > 0 && units <= 128) {
+    const double w = static_cast<double>(D) / 576.0;
+    const double head = 5.0 + 4.5 * w, tile = 0.35 + 0.75 * w;  // us
+    const double whole = head + tile * static_cast<double>(tiles);
+    double best = 0.75 * whole;
+    for (int64_t n = 2; n <= 32 && n <= tiles && units * n <= 256; ++n) {
+      const int64_t per = (tiles + n - 1) / n;
+      const double mb = static_cast<double>(units * n * 64 * D * 4) * 1e-6;
+      const double cost = head + tile * static_cast<double>(per) + 7.0 + 0.6 * mb;
+      if (cost < best) {
+        best = cost;
+        p.mode = ATTN_SPLIT;
+        p.splits = static_cast<int>((tiles + per - 1) / per);
+        p.span = static_cast<int>(per * kAttnTK);
+      }
+    }
+    if (p.mode == ATTN_SPLIT) p.bytes = units * p.splits * 64 * (D * 4 + 8);
+  }
+  return p;
+}
+
+template <int D, int MODE>
+static int launch_attn_mode(const SparseAttnArgs& a, hipStream_t st) {
+  constexpr int R = MODE == ATTN_ROWS && D >= 512 ? kAttnManyRows : 1;
+  const int64_t nblk = static_cast<int64_t>(a.B) * ((a.S + R - 1) / R) * a.HG * a.splits;
   if (nblk > 0x7fffffffLL) return set_error(SI_ERR_UNSUPPORTED, "grid too large");
   const dim3 grid(static_cast<unsigned>(nblk)), block(kAttnThreads);
   if (a.kv2) {  // (int32 indices: the CSA / HCA rows)
-    if (a.f16) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, true, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, false, true>), grid, block, 0, st, a);
+    if (a.f16) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, true, true, MODE>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, false, true, MODE>), grid, block, 0, st, a);
   } else if (a.f16) {
-    if (a.idx64) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, true, true, false>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, true, false>), grid, block, 0, st, a);
+    if (a.idx64) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, true, true, false, MODE>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, true, false, MODE>), grid, block, 0, st, a);
   } else {
-    if (a.idx64) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, true, false, false>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, false, false>), grid, block, 0, st, a);
+    if (a.idx64) hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, true, false, false, MODE>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((sparse_attn_fwd_kernel<D, false, false, false, MODE>), grid, block, 0, st, a);
   }
-  return check_launch("sparse_attn_fwd_kernel");
+  const int rc = check_launch("sparse_attn_fwd_kernel");
+  if (rc || MODE != ATTN_SPLIT) return rc;
+  const int64_t items = static_cast<int64_t>(a.B) * a.S * a.H * (D / 4);
+  const dim3 cgrid(static_cast<unsigned>((items + 255) / 256));
+  if (a.f16) hipLaunchKernelGGL(sparse_attn_combine_kernel<true>, cgrid, dim3(256), 0, st, a, D);
+  else hipLaunchKernelGGL(sparse_attn_combine_kernel<false>, cgrid, dim3(256), 0, st, a, D);
+  return check_launch("sparse_attn_combine_kernel");
+}
+
+template <int D>
+static int launch_attn(const SparseAttnArgs& a, int mode, hipStream_t st) {
+  if (mode == ATTN_SPLIT) return launch_attn_mode<D, ATTN_SPLIT>(a, st);
+  if constexpr (D >= 512) {
+    if (mode == ATTN_ROW) return launch_attn_mode<D, ATTN_ROW>(a, st);
+  }
+  return launch_attn_mode<D, ATTN_ROWS>(a, st);
 }
 
 }  // namespace si
@@ -702,7 +855,9 @@ static int sparse_attn_fwd_entry(const void* q, const int64_t* q_strides, const 
                                  const int64_t* idx_strides, int64_t B, int64_t S, int64_t H, int64_t D, int64_t K,
                                  float softmax_scale, int qkv_dtype, void* o, const int64_t* o_strides, float* lse,
                                  const int64_t* lse_strides, const int32_t* row_len, const int64_t* row_len_strides,
-                                 void* stream) {
+                                 void* scratch, int64_t scratch_bytes, void* stream) {
+  if (scratch && (reinterpret_cast<uintptr_t>(scratch) & 15))
+    return set_error(SI_ERR_INVALID, "scratch must be 16-byte aligned");
   if (row_len && !row_len_strides) return set_error(SI_ERR_INVALID, "null row_len strides");
   if (qkv_dtype != SI_DTYPE_BF16 && qkv_dtype != SI_DTYPE_F16)
     return set_error(SI_ERR_INVALID, "qkv_dtype must be SI_DTYPE_BF16 (0) or SI_DTYPE_F16 (1)");
@@ -767,14 +922,22 @@ static int sparse_attn_fwd_entry(const void* q, const int64_t* q_strides, const 
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.f16 = qkv_dtype == SI_DTYPE_F16 ? 1 : 0;
   if (a.B == 0 || a.S == 0) return SI_OK;
+  AttnPlan p = attn_plan(B, S, H, D, N_kv > 0 ? K : 0);
+  if (p.mode == ATTN_SPLIT && (!scratch || scratch_bytes < p.bytes)) p = AttnPlan{D >= 512 ? ATTN_ROW : ATTN_ROWS, 1, 0, 0};
+  a.splits = p.splits;
+  a.span = p.span;
+  if (p.mode == ATTN_SPLIT) {
+    a.part_o = static_cast<float*>(scratch);
+    a.part_ml = reinterpret_cast<float2*>(a.part_o + B * S * a.HG * p.splits * 64 * D);
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (D) {
-    case 32: return launch_attn<32>(a, st);
-    case 64: return launch_attn<64>(a, st);
-    case 128: return launch_attn<128>(a, st);
-    case 256: return launch_attn<256>(a, st);
-    case 512: return launch_attn<512>(a, st);
-    case 576: return launch_attn<576>(a, st);
+    case 32: return launch_attn<32>(a, p.mode, st);
+    case 64: return launch_attn<64>(a, p.mode, st);
+    case 128: return launch_attn<128>(a, p.mode, st);
+    case 256: return launch_attn<256>(a, p.mode, st);
+    case 512: return launch_attn<512>(a, p.mode, st);
+    case 576: return launch_attn<576>(a, p.mode, st);
     default:
       return set_error(SI_ERR_UNSUPPORTED,
                        "unsupported head dim D=" + std::to_string(D) + " (supported: 32, 64, 128, 256, 512, 576)");
@@ -789,7 +952,30 @@ extern "C" int si_sparse_attn_fwd_ragged(const void* q, const int64_t* q_strides
                                          const int32_t* row_len, const int64_t* row_len_strides, void* stream) {
   return sparse_attn_fwd_entry(q, q_strides, kv, kv_strides, N_kv, nullptr, nullptr, 0, attn_sink, topk_idxs,
                                idx_is_i64, idx_strides, B, S, H, D, K, softmax_scale, qkv_dtype, o, o_strides, lse,
-                               lse_strides, row_len, row_len_strides, stream);
+                               lse_strides, row_len, row_len_strides, nullptr, 0, stream);
+}
+
+extern "C" int64_t si_sparse_attn_fwd_scratch_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int64_t K) {
+  const int64_t lim = 0x7fffffff;
+  if (B <= 0 || S <= 0 || H <= 0 || K <= 0 || B > lim || S > lim || H > lim || K > lim) return 0;
+  if (D != 32 && D != 64 && D != 128 && D != 256 && D != 512 && D != 576) return 0;
+  return attn_plan(B, S, H, D, K).bytes;
+}
+
+extern "C" int si_sparse_attn_fwd_scratch(const void* q, const int64_t* q_strides, const void* kv,
+                                          const int64_t* kv_strides, int64_t N_kv, const void* kv2,
+                                          const int64_t* kv2_strides, int64_t N_kv2, const float* attn_sink,
+                                          const void* topk_idxs, int idx_is_i64, const int64_t* idx_strides, int64_t B,
+                                          int64_t S, int64_t H, int64_t D, int64_t K, float softmax_scale,
+                                          int qkv_dtype, void* o, const int64_t* o_strides, float* lse,
+                                          const int64_t* lse_strides, const int32_t* row_len,
+                                          const int64_t* row_len_strides, void* scratch, int64_t scratch_bytes,
+                                          void* stream) {
+  if (B > 0 && S > 0 && N_kv2 > 0 && !kv2) return set_error(SI_ERR_INVALID, "null pointer argument");
+  return sparse_attn_fwd_entry(q, q_strides, kv, kv_strides, N_kv, N_kv2 > 0 ? kv2 : nullptr, kv2_strides, N_kv2,
+                               attn_sink, topk_idxs, idx_is_i64, idx_strides, B, S, H, D, K, softmax_scale, qkv_dtype,
+                               o, o_strides, lse, lse_strides, row_len, row_len_strides, scratch, scratch_bytes,
+                               stream);
 }
 
 extern "C" int si_sparse_attn_fwd_kv2(const void* q, const int64_t* q_strides, const void* kv,
@@ -803,7 +989,7 @@ extern "C" int si_sparse_attn_fwd_kv2(const void* q, const int64_t* q_strides, c
   // (a null kv2 with no rows is the one-tensor case)
   return sparse_attn_fwd_entry(q, q_strides, kv, kv_strides, N_kv, N_kv2 > 0 ? kv2 : nullptr, kv2_strides, N_kv2,
                                attn_sink, topk_idxs, 0, idx_strides, B, S, H, D, K, softmax_scale, qkv_dtype, o,
-                               o_strides, lse, lse_strides, row_len, row_len_strides, stream);
+                               o_strides, lse, lse_strides, row_len, row_len_strides, nullptr, 0, stream);
 }
 
 extern "C" int si_sparse_attn_fwd(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,

@@ -106,13 +106,7 @@ def _topk_launch(q, k_idx, weights, top_k, causal_mask, causal_ratio):
     L = _lib.load()
     with torch.cuda.device(q.device):
         # Few query rows over many keys: a score scratch lets the call use the whole GPU.
-        nscratch = L.si_indexer_topk_scratch_bytes(B, S, T, H_I, D_I, top_k, ratio)
-        scratch = None
-        if nscratch:
-            try:
-                scratch = torch.empty((nscratch,), dtype=torch.uint8, device=q.device)
-            except torch.OutOfMemoryError:
-                nscratch = 0  # the kernel that needs none
+        scratch, nscratch = _lib.scratch(L.si_indexer_topk_scratch_bytes(B, S, T, H_I, D_I, top_k, ratio), q.device)
         rc = L.si_indexer_topk_scratch(
             q.data_ptr(), _lib.strides(q), k_idx.data_ptr(), _lib.strides(k_idx),
             weights.data_ptr(), 1 if weights.dtype == torch.bfloat16 else 0, _lib.strides(weights),

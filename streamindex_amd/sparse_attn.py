@@ -103,12 +103,14 @@ def sparse_attn_fwd(
     lse = torch.empty((B, S, H), dtype=torch.float32, device=q.device)
     L = _lib.load()
     with torch.cuda.device(q.device):
-        rc = L.si_sparse_attn_fwd_ragged(
-            q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), attn_sink.data_ptr(),
+        scratch, nscratch = _lib.scratch(L.si_sparse_attn_fwd_scratch_bytes(B, S, H, D, K), q.device)
+        rc = L.si_sparse_attn_fwd_scratch(
+            q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), N_kv, None, None, 0, attn_sink.data_ptr(),
             topk_idxs.data_ptr(), 1 if topk_idxs.dtype == torch.int64 else 0, _lib.strides(topk_idxs),
-            B, S, H, D, N_kv, K, float(softmax_scale), _lib.qkv_dtype(q), o.data_ptr(), _lib.strides(o),
+            B, S, H, D, K, float(softmax_scale), _lib.qkv_dtype(q), o.data_ptr(), _lib.strides(o),
             lse.data_ptr(), _lib.strides(lse), None if row_len is None else row_len.data_ptr(),
-            None if row_len is None else _lib.strides(row_len), _lib.stream_ptr(q.device))
+            None if row_len is None else _lib.strides(row_len), None if scratch is None else scratch.data_ptr(),
+            nscratch, _lib.stream_ptr(q.device))
     _lib.check(rc)
     return o, lse
 
@@ -160,12 +162,14 @@ def sparse_attn_fwd_kv2(
     lse = torch.empty((B, S, H), dtype=torch.float32, device=q.device)
     L = _lib.load()
     with torch.cuda.device(q.device):
-        rc = L.si_sparse_attn_fwd_kv2(
+        scratch, nscratch = _lib.scratch(L.si_sparse_attn_fwd_scratch_bytes(B, S, H, D, K), q.device)
+        rc = L.si_sparse_attn_fwd_scratch(
             q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), N1, kv2.data_ptr(), _lib.strides(kv2),
-            N2, attn_sink.data_ptr(), topk_idxs.data_ptr(), _lib.strides(topk_idxs), B, S, H, D, K,
+            N2, attn_sink.data_ptr(), topk_idxs.data_ptr(), 0, _lib.strides(topk_idxs), B, S, H, D, K,
             float(softmax_scale), _lib.qkv_dtype(q), o.data_ptr(), _lib.strides(o), lse.data_ptr(),
             _lib.strides(lse), None if row_len is None else row_len.data_ptr(),
-            None if row_len is None else _lib.strides(row_len), _lib.stream_ptr(q.device))
+            None if row_len is None else _lib.strides(row_len), None if scratch is None else scratch.data_ptr(),
+            nscratch, _lib.stream_ptr(q.device))
     _lib.check(rc)
     return o, lse
 
