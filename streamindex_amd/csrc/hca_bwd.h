@@ -1,0 +1,486 @@
+// Backward of the HCA composition (included by sparse_attn_bwd.hip).
+//
+// HCA's keys are not scattered: query s attends to the window s-n_win+1 .. s
+// and to every compressed entry i < (s+1)/m.  The general backward writes one
+// dkv row per (query, slot) and sorts and sums them by key; here 64 keys and a
+// block of consecutive queries meet in one workgroup, which sums their dkv in
+// MFMA accumulators, so nothing is written per pair:
+//   1. hca_bwd_idx_kernel: index rows whose window part starts at a multiple of
+//      32 keys, so that slot tile i of query s holds the aligned key tile
+//      (s-n_win+1)/32 + i whatever s is.
+//   2. sparse_attn_bwd_rows_kernel on those rows: dq, dsink terms, and P / dS of
+//      every tile (8 KiB each) in its register layout.
+//   3. hca_bwd_dkv_kernel: per (64 keys, RB query rows) the sum over the rows'
+//      heads of dS q + P dO, fp32, to a partial buffer.
+//   4. hca_bwd_reduce_kernel: each key's partials in block order.
+// Every sum has a fixed order, so repeated calls are bit-identical.
+//
+// Bound: step 2 (its gathers and coefficients) and step 3's copies: a row's Q
+// and dO come through LDS once per 64-key group it meets (4 to 5 at S = 16K),
+// 32 heads at a time so that the next half is copied while one is multiplied.
+// Measured at S = 16,384, 64 heads, D = 576, n_win = m = 128: rows 1.80,
+// dkv 1.55, reduction 0.07 ms, against 1.76 + 1.45 + 1.26 + 0.11 ms (rows, dkv
+// rows, reduction, sort) of the general backward over 3.2M pairs; forward and
+// backward 5.51 -> 4.4 ms.
+#pragma once
+
+namespace si {
+
+struct HcaBwdArgs {
+  int n_win, m, T;
+  int wtiles;      // 32-key window tiles of an index row
+  int RB;          // query rows of a block (a multiple of 32)
+  int b0, nb;      // batches of this chunk
+  int s0, s1;      // query rows of this chunk (s0 a multiple of RB)
+  int GW, ncg;     // window / compressed 64-key groups of a block
+  float* part;     // [nb, blocks, GW + ncg, 64, D]
+  float* acc;      // [B, N, D] fp32 sums of the earlier chunks
+  uint16_t* dkv;   // [B, N, D]
+  int64_t dsb, dsn;
+  int first, last;  // first / last chunk of the batch
+};
+
+// First 64-key window group that row block blk touches (keys below 0 count).
+__device__ __forceinline__ int hca_group_lo(const HcaBwdArgs& h, int blk) { return (blk * h.RB - h.n_win + 1) >> 6; }
+
+// Query rows of (block, group j): the block's rows inside the chunk that have a
+// key of the group.
+__device__ __forceinline__ void hca_item_rows(const HcaBwdArgs& h, int blk, int j, int& r0, int& r1) {
+  r0 = blk * h.RB > h.s0 ? blk * h.RB : h.s0;
+  r1 = (blk + 1) * h.RB < h.s1 ? (blk + 1) * h.RB : h.s1;
+  if (j < h.GW) {
+    const int kg = hca_group_lo(h, blk) + j;
+    const int lo = 64 * kg, hi = 64 * kg + 63 + h.n_win;  // rows lo .. hi-1 see keys 64 kg .. 64 kg + 63
+    if (kg < 0) r1 = r0;
+    r0 = r0 > lo ? r0 : lo;
+    r1 = r1 < hi ? r1 : hi;
+  } else {
+    const int64_t lo = static_cast<int64_t>(h.m) * (64 * (j - h.GW) + 1) - 1;
+    if (r0 < lo) r0 = lo < r1 ? static_cast<int>(lo) : r1;
+  }
+}
+
+// Index rows [S, 32 wtiles + T] and their used lengths [S], shared by all
+// batches: window column j of query s holds key 32 floor((s-n_win+1)/32) + j
+// where that lies in the window, then compressed entry i as S + i, else -1.
+__global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t* row_len, int S, int n_win, int T, int m,
+                                                          int wtiles) {
+  const int s = blockIdx.x;
+  const int K = 32 * wtiles + T;
+  const int first = s - n_win + 1;
+  const int base = (first >> 5) * 32;
+  const int legal = (s + 1) / m < T ? (s + 1) / m : T;
+  for (int j = threadIdx.x; j < K; j += 256) {
+    int v;
+    if (j < 32 * wtiles) {
+      const int t = base + j;
+      v = t >= 0 && t >= first && t <= s ? t : -1;
+    } else {
+      const int i = j - 32 * wtiles;
+      v = i < legal ? S + i : -1;
+    }
+    idx[static_cast<int64_t>(s) * K + j] = v;
+  }
+  if (threadIdx.x == 0) row_len[s] = 32 * wtiles + legal;
+}
+
+template <int D>
+struct HcaDkvShape {
+  static constexpr int CPR = D / 8;
+  static constexpr int CPP = CPR + 2;          // chunks per LDS row: padded as in DkvShape (conflict-free transposing reads)
+  static constexpr int QROW = CPP * 16;
+  static constexpr int HALF = 32 * QROW;       // 32 heads of Q or of dO
+  static constexpr int BUF = 2 * HALF;         // Q then dO
+  static constexpr int NW = 8;                      // waves, two per SIMD
+  static constexpr int COPIES = 2 * 32 * CPP / 64;  // 64-lane copies of a stage
+  static constexpr int CPW = (COPIES + NW - 1) / NW;  // copies per wave
+  // 16-dimension blocks: MBW each for waves 0..3, the rest in equal shares for
+  // waves 4..7, so that the two waves of a SIMD hold MBT / 4 together.
+  static constexpr int MBT = D / 16;
+  static constexpr int MBW = (MBT + 7) / 8;
+  static constexpr int MBW2 = MBT > 4 * MBW ? (MBT - 4 * MBW) / 4 : 0;
+  static_assert(MBT <= 4 * MBW || (MBT - 4 * MBW) % 4 == 0, "blocks of waves 4..7");
+  // Coefficients: [tile][P, dS][producer wave][4-key group][head][16 bytes], the
+  // key groups 320 bytes apart (256 would put a transposing read's four in one bank)
+  static constexpr int CG = 320;
+  static constexpr int CW4 = 4 * CG;
+  static constexpr int COEF = 2 * 2 * 2 * CW4;
+};
+
+// 16 bytes per lane from memory to LDS (64 lanes: consecutive slots from dst).
+__device__ __forceinline__ void hca_copy16(const uint16_t* src, char* dst) {
+  __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 16, 0, 0);
+}
+
+// dkv^T [D x 64 keys] += [Q^T | dO^T] [D x 64] . [dS; P] [64 x 64 keys] per stage
+// (one query row, 32 heads), the operands as in sparse_attn_bwd_dkv_rows_kernel.
+// Two waves per SIMD: one's copies, waits and fragment reads run beside the
+// other's MFMAs.  Bound: the copies, 16 bytes a clock and CU (8.7 TB/s from the
+// L2; the same rows from L2 throughout take as long, without the copies the
+// kernel takes 0.83 instead of 1.55 ms; spreading them over the blocks, or
+// touching the lines two rows ahead, changed nothing).
+template <int D, bool F16>
+__global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdArgs h) {
+  using HS = HcaDkvShape<D>;
+  constexpr int MBW = HS::MBW;
+  __shared__ __attribute__((aligned(16))) char qd_lds[2 * HS::BUF];
+  __shared__ __attribute__((aligned(16))) char coef_lds[HS::COEF];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __builtin_assume(wave >= 0 && wave < HS::NW);
+  const int g = lane >> 4;
+  const int i16 = lane & 15;
+  const int per = h.GW + h.ncg;
+  const int blk0 = h.s0 / h.RB;
+  const int nblk = (h.s1 + h.RB - 1) / h.RB - blk0;
+  const int item = xcd_block_order();  // neighbouring items share their rows' Q and dO
+  const int j = item % per;
+  const int blk = blk0 + (item / per) % nblk;
+  const int b = h.b0 + item / (per * nblk);
+  int r0, r1;
+  hca_item_rows(h, blk, j, r0, r1);
+  if (r0 >= r1) return;
+  const bool window = j < h.GW;
+  const int kt = 2 * (window ? hca_group_lo(h, blk) + j : j - h.GW);  // first 32-key tile of the group
+  const int blk_lo = wave < 4 ? wave * MBW : 4 * MBW + (wave - 4) * HS::MBW2;  // this wave's dimension blocks
+
+  // Copies of a stage: LDS chunk e (16 bytes) is chunk e % CPP of head
+  // (e / CPP) % 32 of Q (e < 32 CPP) or dO; the pad chunks re-read chunk 0.
+  // Copy n = NW i + wave is wholly one of the two (32 CPP is a multiple of 64).
+  int voff[HS::CPW];  // byte offset from the stage's first head
+#pragma unroll
+  for (int i = 0; i < HS::CPW; ++i) {
+    const int n = i * HS::NW + wave;
+    const int e = n * 64 + lane;
+    const int c = e % HS::CPP;
+    voff[i] = static_cast<int>(((e / HS::CPP) % 32) * (n < HS::COPIES / 2 ? a.qsh : a.gsh) + (c < HS::CPR ? c : 0) * 8) * 2;
+  }
+  struct Stage {
+    int s, hg, half;
+  };
+  auto next = [&](Stage x) {
+    if (x.half == 0) return Stage{x.s, x.hg, 1};
+    return x.hg + 1 < a.HG ? Stage{x.s, x.hg + 1, 0} : Stage{x.s + 1, 0, 0};
+  };
+  auto copy_stage = [&](const Stage& x, int buf) {
+    const int h0 = x.hg * 64 + x.half * 32;
+    const char* qs = reinterpret_cast<const char*>(a.q + b * a.qsb + static_cast<int64_t>(x.s) * a.qss + h0 * a.qsh);
+    const char* gs = reinterpret_cast<const char*>(a.dout + b * a.gsb + static_cast<int64_t>(x.s) * a.gss + h0 * a.gsh);
+    char* dst = qd_lds + buf * HS::BUF;
+    const bool whole = h0 + 32 <= a.H;
+#pragma unroll
+    for (int i = 0; i < HS::CPW; ++i) {
+      const int n = i * HS::NW + wave;
+      if (n < HS::COPIES) {
+        const bool isq = n < HS::COPIES / 2;
+        int off = voff[i];
+        if (!whole) {
+          // heads past H re-read the last one below it, or head H-1 (their P and
+          // dS are 0): step back whole heads
+          const int e = n * 64 + lane;
+          const int hd = (e / HS::CPP) % 32;
+          const int over = h0 + hd - (a.H - 1);
+          if (over > 0) off -= over * static_cast<int>(isq ? a.qsh : a.gsh) * 2;
+        }
+        hca_copy16(reinterpret_cast<const uint16_t*>((isq ? qs : gs) + off), dst + n * 1024);
+      }
+    }
+  };
+  // Coefficients of a stage: tiles kt and kt+1, 32 heads (two producer waves),
+  // by waves 0..3; zero where the query row has no such tile.
+  const int64_t nr = h.s1 - h.s0;
+  u32x4 cf[2];
+  auto load_coef = [&](const Stage& x) {
+    if (wave >= 4) return;
+    const int64_t lrow = (b - h.b0) * nr + (x.s - h.s0);
+    const uint16_t* row = a.coef + (lrow * a.HG + x.hg) * a.ntiles * kCoefTile;
+    const int t = threadIdx.x;  // [P, dS][producer wave][lane]
+    const int off = ((t >> 7) * 4 + 2 * x.half + ((t >> 6) & 1)) * 512 + (t & 63) * 8;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      int ti = kt + k;
+      bool ok;
+      if (window) {
+        ti -= (x.s - h.n_win + 1) >> 5;
+        ok = ti >= 0 && ti < h.wtiles;
+      } else {
+        ok = static_cast<int64_t>(h.m) * (ti * 32 + 1) <= x.s + 1 && ti * 32 < h.T;  // its first entry is legal
+        ti += h.wtiles;
+      }
+      cf[k] = ok ? *reinterpret_cast<const u32x4*>(row + static_cast<int64_t>(ti) * kCoefTile + off) : u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+
+  const uint32_t qd0 = lds_addr(qd_lds) + (8 * g + (i16 >> 2)) * HS::QROW + 8 * (i16 & 3) + blk_lo * 32;
+  const int bh = 8 * g + (i16 >> 2);  // head of the 32
+  const uint32_t cf0 = lds_addr(coef_lds) + (bh >> 4) * HS::CW4 + (i16 & 3) * HS::CG + (bh & 15) * 16;
+  const int cst = ((threadIdx.x >> 6) & 3) * HS::CW4 + (lane >> 4) * HS::CG + (lane & 15) * 16;  // where load_coef's words go
+
+  // The stages with NB dimension blocks (a compile-time count: LDS reads in
+  // flight must not cross control flow, where their registers could be copied
+  // before the data lands).
+  auto stages = [&](auto NBC) {
+    constexpr int NB = decltype(NBC)::value;
+    f32x4 acc[NB > 0 ? NB : 1][4];
+#pragma unroll
+    for (int m = 0; m < NB; ++m)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Stage cur{r0, 0, 0};
+    copy_stage(cur, 0);
+    load_coef(cur);
+    int buf = 0;
+    for (; cur.s < r1; buf ^= 1) {
+      __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));  // this stage's copies and coefficients landed (issued a stage ago)
+      if (wave < 4) {
+        *reinterpret_cast<u32x4*>(coef_lds + cst) = cf[0];
+        *reinterpret_cast<u32x4*>(coef_lds + 4 * HS::CW4 + cst) = cf[1];
+      }
+      attn_tile_barrier();
+      // (the other buffer was last read in the previous stage, which every wave has left)
+      cur = next(cur);
+      if (cur.s < r1) {
+        copy_stage(cur, buf ^ 1);
+        load_coef(cur);
+      }
+      if constexpr (NB > 0) {
+        // k-step 0: dS of the 32 heads against Q; 1: P against dO.  Key blocks
+        // nb: 16 (nb & 1) of tile nb >> 1.
+        v4i16 blo[2][4], bhi[2][4];
+        attn_static_for<0, 2>([&](auto KC) {
+          attn_static_for<0, 4>([&](auto NC) {
+            constexpr int ks = decltype(KC)::value;
+            constexpr int nb = decltype(NC)::value;
+            constexpr int off = (nb >> 1) * 4 * HS::CW4 + (ks == 0 ? 2 * HS::CW4 : 0) + 8 * (nb & 1);
+            blo[ks][nb] = tr_read<off>(cf0);
+            bhi[ks][nb] = tr_read<off + 64>(cf0);
+          });
+        });
+        const uint32_t qa = qd0 + buf * HS::BUF;
+        v4i16 alo[2][2], ahi[2][2];
+        auto a_read = [&](auto JC) {
+          constexpr int m = decltype(JC)::value;
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            alo[m & 1][ks] = tr_read<m * 32>(qa + ks * HS::HALF);
+            ahi[m & 1][ks] = tr_read<m * 32 + 4 * HS::QROW>(qa + ks * HS::HALF);
+          }
+        };
+        a_read(std::integral_constant<int, 0>{});
+        lds_wait_n<4>();
+        bf16x8 bfr[2][4];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int nb = 0; nb < 4; ++nb) {
+            reg_tie(blo[ks][nb]);
+            reg_tie(bhi[ks][nb]);
+            bfr[ks][nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[ks][nb], bhi[ks][nb], 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+        attn_static_for<0, NB>([&](auto JC) {
+          constexpr int m = decltype(JC)::value;
+          if constexpr (m + 1 < NB) {
+            a_read(std::integral_constant<int, m + 1>{});
+            lds_wait_n<4>();
+          } else {
+            lds_wait_n<0>();
+          }
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            reg_tie(alo[m & 1][ks]);
+            reg_tie(ahi[m & 1][ks]);
+          }
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo[m & 1][ks], ahi[m & 1][ks], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) acc[m][nb] = mfma16x16x32<F16>(af, bfr[ks][nb], acc[m][nb]);
+          }
+        });
+      }
+      attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
+    }
+#pragma unroll
+    for (int m = 0; m < NB; ++m) {
+      mfma_result_fence(acc[m][0], acc[m][1]);
+      mfma_result_fence(acc[m][2], acc[m][3]);
+    }
+    // lane (key 16 nb + i16 of the group, g) holds dimensions 16 mbi + 4 g + 0..3
+    float* out = h.part + static_cast<int64_t>(item) * 64 * D;
+#pragma unroll
+    for (int m = 0; m < NB; ++m) {
+      if (blk_lo + m < HS::MBT) {  // (at D = 32 waves 2 and 3 hold no block of the row)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb)
+          *reinterpret_cast<f32x4*>(out + (nb * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = acc[m][nb];
+      }
+    }
+  };
+  if (wave < 4) stages(std::integral_constant<int, MBW>{});
+  else stages(std::integral_constant<int, HS::MBW2>{});
+}
+
+// dkv of one key from its partials (blocks in order), the sums of the earlier
+// chunks first.  Keys without a partial in a middle chunk keep their sum.
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void hca_bwd_reduce_kernel(HcaBwdArgs h, int S) {
+  const int N = S + h.T;
+  const int n = static_cast<int>(blockIdx.x) % N;
+  const int b = h.b0 + static_cast<int>(blockIdx.x) / N;
+  const int d = static_cast<int>(threadIdx.x) * 4;
+  const int per = h.GW + h.ncg;
+  const int blk0 = h.s0 / h.RB;
+  const int nblk = (h.s1 + h.RB - 1) / h.RB - blk0;
+  const bool window = n < S;
+  const int grp = (window ? n : n - S) >> 6;
+  const int64_t lo = window ? 64 * grp : static_cast<int64_t>(h.m) * (64 * grp + 1) - 1;
+  const int64_t hi = window ? 64 * grp + 63 + h.n_win : h.s1;
+  int64_t from = lo > h.s0 ? lo : h.s0, to = hi < h.s1 ? hi : h.s1;  // rows with a key of the group
+  if (window ? h.GW == 0 : grp >= h.ncg) to = from;
+  if (from >= to && !h.first && !h.last) return;
+  if (d >= D) return;
+  f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+  float* acc = h.acc + (static_cast<int64_t>(b) * N + n) * D + d;
+  if (!h.first) sum = *reinterpret_cast<const f32x4*>(acc);
+  if (from < to) {
+    const int q0 = static_cast<int>(from) / h.RB, q1 = static_cast<int>(to - 1) / h.RB;  // inclusive
+    auto part = [&](int q) {
+      const int j = window ? grp - hca_group_lo(h, q) : h.GW + grp;
+      const int64_t item = (static_cast<int64_t>(b - h.b0) * nblk + (q - blk0)) * per + j;
+      return *reinterpret_cast<const f32x4*>(h.part + (item * 64 + ((window ? n : n - S) & 63)) * D + d);
+    };
+    for (int q = q0; q <= q1; q += 8) {
+      f32x4 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part(q + u <= q1 ? q + u : q1);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sum[c] += q + u <= q1 ? v[u][c] : 0.f;
+    }
+  }
+  if (!h.last) {
+    *reinterpret_cast<f32x4*>(acc) = sum;
+  } else {
+    uint2 w;
+    w.x = pack2<F16>(sum[0], sum[1]);
+    w.y = pack2<F16>(sum[2], sum[3]);
+    *reinterpret_cast<uint2*>(h.dkv + b * h.dsb + static_cast<int64_t>(n) * h.dsn + d) = w;
+  }
+}
+
+// ---- host side ----------------------------------------------------------------
+struct HcaPlan {
+  int64_t rows;  // query rows of a chunk (a multiple of RB, or S)
+  int64_t nb;    // batches of a chunk (all of them, or 1 where a batch takes several chunks)
+  int RB, wtiles, ntiles, GW, ncg;
+  size_t dsink_rows, acc, idx, row_len, coef, part, total;
+};
+
+static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, int RB, int64_t rows,
+                         int64_t nb, HcaPlan* p) {
+  const int64_t HG = (H + 63) / 64;
+  p->rows = rows;
+  p->nb = nb;
+  p->RB = RB;
+  p->wtiles = n_win > 0 ? static_cast<int>((n_win + 31 + 31) / 32) : 0;
+  p->ntiles = p->wtiles + static_cast<int>((T + 31) / 32);
+  p->GW = n_win > 0 ? static_cast<int>((RB + n_win - 2) / 64 + 2) : 0;
+  p->ncg = static_cast<int>((T + 63) / 64);
+  size_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const size_t at = off;
+    off = (off + static_cast<size_t>(bytes) + 255) & ~static_cast<size_t>(255);
+    return at;
+  };
+  const int64_t blocks = (rows + RB - 1) / RB;
+  p->dsink_rows = take(B * S * 64 * HG * 4);
+  p->acc = take(rows < S ? B * (S + T) * D * 4 : 0);
+  p->idx = take(S * (32 * p->wtiles + T) * 4);
+  p->row_len = take(S * 4);
+  p->coef = take(nb * rows * HG * p->ntiles * kCoefTile * 2);
+  p->part = take(nb * blocks * (p->GW + p->ncg) * 64 * D * 4);
+  p->total = off;
+}
+
+// The fewest chunks whose plan fits `bytes`; false when none does.  Row blocks
+// of 128 (fewer partials), smaller where that leaves CUs idle.
+static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, size_t bytes, HcaPlan* p) {
+  for (int RB = 64; RB >= 32; RB /= 2) {
+    hca_plan_for(B, S, H, D, n_win, T, RB, S, B, p);
+    if (RB == 32 || B * ((S + RB - 1) / RB) * (p->GW + p->ncg) >= 1024) break;
+  }
+  if (p->total <= bytes) return true;
+  const int RB = p->RB;
+  int64_t lo = 0, hi = (S + RB - 1) / RB;  // chunks of `lo` row blocks fit
+  while (hi - lo > 1) {
+    const int64_t mid = (lo + hi) / 2;
+    hca_plan_for(B, S, H, D, n_win, T, RB, mid * RB, 1, p);
+    if (p->total <= bytes) lo = mid; else hi = mid;
+  }
+  if (lo == 0) {
+    hca_plan_for(B, S, H, D, n_win, T, RB, S, 1, p);  // one chunk per batch
+    return p->total <= bytes;
+  }
+  hca_plan_for(B, S, H, D, n_win, T, RB, lo * RB, 1, p);
+  return true;
+}
+
+template <int D, bool F16>
+static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs h, float* dsink, hipStream_t st) {
+  const int S = a.S;
+  const int K = 32 * pl.wtiles + h.T;
+  int32_t* idx = reinterpret_cast<int32_t*>(ws + pl.idx);
+  int32_t* row_len = reinterpret_cast<int32_t*>(ws + pl.row_len);
+  int rc;
+  hipLaunchKernelGGL(hca_bwd_idx_kernel, dim3(static_cast<unsigned>(S)), dim3(256), 0, st, idx, row_len, S, h.n_win, h.T,
+                     h.m, pl.wtiles);
+  if ((rc = check_launch("hca_bwd_idx_kernel"))) return rc;
+  a.idx = idx;
+  a.isb = 0;
+  a.iss = K;
+  a.isk = 1;
+  a.row_len = row_len;
+  a.rlsb = 0;
+  a.rlss = 1;
+  a.K = K;
+  a.ntiles = pl.ntiles;
+  a.dsink_rows = reinterpret_cast<float*>(ws + pl.dsink_rows);
+  a.coef = reinterpret_cast<uint16_t*>(ws + pl.coef);
+  h.wtiles = pl.wtiles;
+  h.RB = pl.RB;
+  h.GW = pl.GW;
+  h.ncg = pl.ncg;
+  h.part = reinterpret_cast<float*>(ws + pl.part);
+  h.acc = reinterpret_cast<float*>(ws + pl.acc);
+  h.nb = static_cast<int>(pl.nb);
+  for (int64_t b0 = 0; b0 < a.B; b0 += pl.nb) {
+    for (int64_t s0 = 0; s0 < S; s0 += pl.rows) {
+      h.b0 = static_cast<int>(b0);
+      h.s0 = static_cast<int>(s0);
+      h.s1 = static_cast<int>(S - s0 < pl.rows ? S : s0 + pl.rows);
+      h.first = s0 == 0;
+      h.last = h.s1 == S;
+      a.row0 = b0 * S + s0;
+      a.nrows = static_cast<int>(pl.nb * (h.s1 - h.s0));
+      const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(a.nrows) * a.HG);
+      hipLaunchKernelGGL((sparse_attn_bwd_rows_kernel<D, false, F16>), dim3(grid), dim3(kBwdThreads), 0, st, a);
+      if ((rc = check_launch("sparse_attn_bwd_rows_kernel"))) return rc;
+      const int64_t blocks = (h.s1 + h.RB - 1) / h.RB - h.s0 / h.RB;
+      const unsigned items = static_cast<unsigned>(pl.nb * blocks * (h.GW + h.ncg));
+      if (items > 0) {
+        hipLaunchKernelGGL((hca_bwd_dkv_kernel<D, F16>), dim3(items), dim3(HcaDkvShape<D>::NW * 64), 0, st, a, h);
+        if ((rc = check_launch("hca_bwd_dkv_kernel"))) return rc;
+      }
+      hipLaunchKernelGGL((hca_bwd_reduce_kernel<D, F16>), dim3(static_cast<unsigned>(pl.nb * (S + h.T))), dim3((D / 4 + 63) / 64 * 64), 0,
+                         st, h, S);
+      if ((rc = check_launch("hca_bwd_reduce_kernel"))) return rc;
+    }
+  }
+  hipLaunchKernelGGL(sparse_attn_bwd_dsink_kernel, dim3(static_cast<unsigned>(a.H)), dim3(256), 0, st, a.dsink_rows,
+                     static_cast<int64_t>(a.B) * S, 64 * a.HG, dsink);
+  return check_launch("sparse_attn_bwd_dsink_kernel");
+}
+
+}  // namespace si

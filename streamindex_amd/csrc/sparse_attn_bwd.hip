@@ -1162,7 +1162,108 @@ static bool bwd_supported_d(int64_t D) {
 
 }  // namespace si
 
+#include "hca_bwd.h"
+
 using namespace si;
+
+static int hca_check(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, int64_t m) {
+  if (B <= 0 || S <= 0 || H <= 0 || D <= 0 || n_win < 0 || T < 0 || m <= 0) return set_error(SI_ERR_INVALID, "bad dimension");
+  if (!bwd_supported_d(D)) return set_error(SI_ERR_UNSUPPORTED, "unsupported head dim D=" + std::to_string(D));
+  const int64_t lim = int64_t{1} << 30;
+  const int64_t HG = (H + 63) / 64;
+  if (S >= lim || n_win >= lim || T >= lim || m >= lim || H >= lim || B * (S + T) >= lim || B * S * HG >= lim ||
+      S * (n_win + T + 64) >= (int64_t{1} << 40) || n_win + T == 0 || m * (T + 64) >= (int64_t{1} << 40))
+    return set_error(SI_ERR_UNSUPPORTED, "HCA backward: shape outside the aligned path");
+  return SI_OK;
+}
+
+extern "C" int64_t si_hca_attn_bwd_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T,
+                                                   int64_t m, int64_t max_bytes) {
+  HcaPlan p{};
+  if (hca_check(B, S, H, D, n_win, T, m) || max_bytes < 0) return -1;
+  if (!hca_plan(B, S, H, D, n_win, T, static_cast<size_t>(max_bytes), &p)) {
+    set_error(SI_ERR_UNSUPPORTED, "HCA backward: no chunk fits the workspace");
+    return -1;
+  }
+  return static_cast<int64_t>(p.total);
+}
+
+extern "C" int si_hca_attn_bwd(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,
+                               const float* attn_sink, const void* o, const int64_t* o_strides, const float* lse,
+                               const int64_t* lse_strides, const void* dout, const int64_t* do_strides, int64_t B,
+                               int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, int64_t m,
+                               float softmax_scale, int qkv_dtype, void* dq, const int64_t* dq_strides, void* dkv,
+                               const int64_t* dkv_strides, float* dsink, void* workspace, int64_t workspace_bytes,
+                               void* stream) {
+  int rc = hca_check(B, S, H, D, n_win, T, m);
+  if (rc) return rc;
+  if (qkv_dtype != SI_DTYPE_BF16 && qkv_dtype != SI_DTYPE_F16)
+    return set_error(SI_ERR_INVALID, "qkv_dtype must be SI_DTYPE_BF16 (0) or SI_DTYPE_F16 (1)");
+  if (!q_strides || !kv_strides || !o_strides || !lse_strides || !do_strides || !dq_strides || !dkv_strides)
+    return set_error(SI_ERR_INVALID, "null stride argument");
+  if (!q || !kv || !attn_sink || !o || !lse || !dout || !dq || !dkv || !dsink || !workspace)
+    return set_error(SI_ERR_INVALID, "null pointer argument");
+  if (q_strides[3] != 1 || kv_strides[2] != 1 || o_strides[3] != 1 || do_strides[3] != 1 || dq_strides[3] != 1 ||
+      dkv_strides[2] != 1)
+    return set_error(SI_ERR_INVALID, "q, kv, o, do, dq and dkv need a contiguous last dimension");
+  if ((q_strides[0] | q_strides[1] | q_strides[2] | kv_strides[0] | kv_strides[1] | o_strides[0] | o_strides[1] |
+       o_strides[2] | do_strides[0] | do_strides[1] | do_strides[2] | dq_strides[0] | dq_strides[1] | dq_strides[2] |
+       dkv_strides[0] | dkv_strides[1]) % 8)
+    return set_error(SI_ERR_INVALID, "strides must be multiples of 8 elements");
+  if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kv) | reinterpret_cast<uintptr_t>(o) |
+       reinterpret_cast<uintptr_t>(dout) | reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dkv) |
+       reinterpret_cast<uintptr_t>(workspace)) & 15)
+    return set_error(SI_ERR_INVALID, "tensors and the workspace must be 16-byte aligned");
+  if (((S + T - 1) * kv_strides[1] + D) / 8 >= (int64_t{1} << 32))
+    return set_error(SI_ERR_UNSUPPORTED, "kv batch larger than 64 GiB");
+  // (head offsets inside a row are 32-bit)
+  if (q_strides[2] < 0 || do_strides[2] < 0 || q_strides[2] >= (int64_t{1} << 24) || do_strides[2] >= (int64_t{1} << 24))
+    return set_error(SI_ERR_UNSUPPORTED, "head stride outside the aligned path");
+  HcaPlan pl{};
+  if (workspace_bytes < 0 || !hca_plan(B, S, H, D, n_win, T, static_cast<size_t>(workspace_bytes), &pl))
+    return set_error(SI_ERR_INVALID, "workspace too small (see si_hca_attn_bwd_workspace_bytes)");
+  AttnBwdArgs a{};
+  a.q = static_cast<const uint16_t*>(q);
+  a.qsb = q_strides[0]; a.qss = q_strides[1]; a.qsh = q_strides[2];
+  a.kv = static_cast<const uint16_t*>(kv);
+  a.kvsb = kv_strides[0]; a.kvsn = kv_strides[1];
+  a.sink = attn_sink;
+  a.o = static_cast<const uint16_t*>(o);
+  a.osb = o_strides[0]; a.oss = o_strides[1]; a.osh = o_strides[2];
+  a.dout = static_cast<const uint16_t*>(dout);
+  a.gsb = do_strides[0]; a.gss = do_strides[1]; a.gsh = do_strides[2];
+  a.lse = lse;
+  a.lsb = lse_strides[0]; a.lss = lse_strides[1]; a.lsh = lse_strides[2];
+  a.dq = static_cast<uint16_t*>(dq);
+  a.dqsb = dq_strides[0]; a.dqss = dq_strides[1]; a.dqsh = dq_strides[2];
+  a.B = static_cast<int>(B); a.S = static_cast<int>(S); a.H = static_cast<int>(H);
+  a.N = static_cast<int>(S + T);
+  a.HG = static_cast<int>((H + 63) / 64);
+  a.scale = softmax_scale;
+  a.scale_log2 = softmax_scale * 1.4426950408889634f;
+  a.f16 = qkv_dtype == SI_DTYPE_F16 ? 1 : 0;
+  HcaBwdArgs h{};
+  h.n_win = static_cast<int>(n_win);
+  h.m = static_cast<int>(m);
+  h.T = static_cast<int>(T);
+  h.dkv = static_cast<uint16_t*>(dkv);
+  h.dsb = dkv_strides[0];
+  h.dsn = dkv_strides[1];
+  char* ws = static_cast<char*>(workspace);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto run = [&](auto DC) {
+    constexpr int DD = decltype(DC)::value;
+    return a.f16 ? launch_hca_bwd<DD, true>(a, pl, ws, h, dsink, st) : launch_hca_bwd<DD, false>(a, pl, ws, h, dsink, st);
+  };
+  switch (D) {
+    case 32: return run(std::integral_constant<int, 32>{});
+    case 64: return run(std::integral_constant<int, 64>{});
+    case 128: return run(std::integral_constant<int, 128>{});
+    case 256: return run(std::integral_constant<int, 256>{});
+    case 512: return run(std::integral_constant<int, 512>{});
+    default: return run(std::integral_constant<int, 576>{});
+  }
+}
 
 extern "C" int64_t si_sparse_attn_bwd_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int64_t N_kv,
                                                       int64_t K, int64_t max_bytes) {

@@ -9,7 +9,9 @@ sparse-attention kernel as CSA.  The index rows are written by one HIP kernel
 arange/where/cat passes.
 
 ``use_triton`` is accepted for compatibility and selects nothing (one HIP
-implementation).  Gradients flow through ``sparse_attn``'s autograd.
+implementation).  The backward knows the rows' structure too: it sums dkv for
+64 keys and a block of queries at a time (``si_hca_attn_bwd``) instead of
+sorting (query, slot) pairs by key.
 """
 
 from __future__ import annotations
@@ -18,8 +20,9 @@ from typing import Optional
 
 import torch
 
+from . import _lib
 from .csa import _launch_hca
-from .sparse_attn import sparse_attn_kv2
+from .sparse_attn import _aligned, _bwd_workspace, sparse_attn_bwd, sparse_attn_fwd_kv2
 
 __all__ = ["flash_hca_forward", "build_hca_topk_idxs", "hca_row_len"]
 
@@ -65,11 +68,58 @@ def flash_hca_forward(
     B, S, n_h, d = q.shape
     n_compressed = kv_compressed.shape[1]
     assert q.is_cuda
-    topk_idxs = build_hca_topk_idxs(B=B, seq_len=S, n_win=n_win, n_compressed=n_compressed, m_prime=m_prime,
-                                    device=q.device)
-    row_len = hca_row_len(B, S, n_win, n_compressed, m_prime, q.device)
-    # the rows index [kv ; kv_compressed]; the kernel reads both in place
-    return sparse_attn_kv2(q, kv, kv_compressed, attn_sink, topk_idxs, softmax_scale, row_len=row_len)
+    return _HcaAttnFunc.apply(q, kv, kv_compressed, attn_sink, softmax_scale, n_win, m_prime)
+
+
+def _rows(B: int, S: int, n_win: int, n_compressed: int, m_prime: int, device):
+    return (build_hca_topk_idxs(B=B, seq_len=S, n_win=n_win, n_compressed=n_compressed, m_prime=m_prime, device=device),
+            hca_row_len(B, S, n_win, n_compressed, m_prime, device))
+
+
+class _HcaAttnFunc(torch.autograd.Function):
+    """HCA attention; the backward rebuilds what it needs of the index rows."""
+
+    @staticmethod
+    def forward(ctx, q, kv, kv_compressed, attn_sink, softmax_scale, n_win, m_prime):
+        topk_idxs, row_len = _rows(q.shape[0], q.shape[1], n_win, kv_compressed.shape[1], m_prime, q.device)
+        # the rows index [kv ; kv_compressed]; the kernel reads both in place
+        o, lse = sparse_attn_fwd_kv2(q, kv, kv_compressed, attn_sink, topk_idxs, softmax_scale, row_len=row_len)
+        ctx.save_for_backward(q, kv, kv_compressed, attn_sink, o, lse)
+        ctx.args = (softmax_scale, n_win, m_prime)
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        q, kv, kv_compressed, attn_sink, o, lse = ctx.saved_tensors
+        dq, dkv, dsink = _hca_attn_bwd(q, torch.cat([kv, kv_compressed], dim=1), attn_sink, o, lse, do.contiguous(),
+                                       kv_compressed.shape[1], *ctx.args)
+        n1 = kv.shape[1]
+        return dq, dkv[:, :n1], dkv[:, n1:], dsink, None, None, None
+
+
+def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_win, m_prime):
+    """``(dq, dkv, dsink)`` for ``kv = [kv ; kv_compressed]``, by ``si_hca_attn_bwd`` where it serves the shape and its
+    workspace fits the backward's cap, else by the general backward over the index rows."""
+    B, S, H, D = q.shape
+    L = _lib.load()
+    with torch.cuda.device(q.device):
+        ws = _bwd_workspace(lambda cap: L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, n_compressed, m_prime, cap),
+                            None, q.device)
+        if ws is None:
+            topk_idxs, row_len = _rows(B, S, n_win, n_compressed, m_prime, q.device)
+            return sparse_attn_bwd(q, kv, attn_sink, topk_idxs, o, lse, do, softmax_scale, row_len=row_len)
+        q, o, do = (t if _aligned(t) and 0 <= t.stride(2) < 1 << 24 else t.contiguous() for t in (q, o, do))
+        attn_sink = attn_sink.contiguous()
+        dq, dkv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(kv)
+        dsink = torch.empty((H,), dtype=torch.float32, device=q.device)
+        rc = L.si_hca_attn_bwd(
+            q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), attn_sink.data_ptr(), o.data_ptr(),
+            _lib.strides(o), lse.data_ptr(), _lib.strides(lse), do.data_ptr(), _lib.strides(do), B, S, H, D, n_win,
+            n_compressed, m_prime, float(D ** -0.5 if softmax_scale is None else softmax_scale), _lib.qkv_dtype(q),
+            dq.data_ptr(), _lib.strides(dq), dkv.data_ptr(), _lib.strides(dkv), dsink.data_ptr(), ws.data_ptr(),
+            ws.numel(), _lib.stream_ptr(q.device))
+    _lib.check(rc)
+    return dq, dkv, dsink
 
 
 def hca_row_len(B: int, S: int, n_win: int, n_compressed: int, m_prime: int, device) -> torch.Tensor:

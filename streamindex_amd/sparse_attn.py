@@ -182,6 +182,32 @@ def sparse_attn_fwd_kv2(
 BWD_WORKSPACE_CAP = 2 << 30
 
 
+def _bwd_workspace(need, workspace_bytes: Optional[int], device: torch.device) -> Optional[torch.Tensor]:
+    """A workspace of ``need(cap)`` bytes, or None where that is negative (no plan fits the cap)."""
+    default_cap = workspace_bytes is None
+    if workspace_bytes is None:
+        # Memory the caching allocator holds but has not handed out counts
+        # as free too: the driver's free figure alone moves with every
+        # segment the allocator maps, and with it the workspace size,
+        # which then misses the cached block and allocates anew.
+        free, _ = torch.cuda.mem_get_info(device)
+        cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+        workspace_bytes = min(BWD_WORKSPACE_CAP, (free + cached) // 4)
+    n = need(int(workspace_bytes))
+    if n < 0:
+        return None
+    try:
+        return torch.empty((max(int(n), 16),), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        if not default_cap:
+            raise
+        # The allocator's unused blocks may be split too finely to hold the
+        # workspace: size it from the driver's free memory alone.
+        free, _ = torch.cuda.mem_get_info(device)
+        n = need(int(min(BWD_WORKSPACE_CAP, free // 4)))
+        return None if n < 0 else torch.empty((max(int(n), 16),), dtype=torch.uint8, device=device)
+
+
 def _aligned(t: torch.Tensor) -> bool:
     return t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
 
@@ -243,30 +269,10 @@ def sparse_attn_bwd(
     dsink = torch.empty((H,), dtype=torch.float32, device=q.device)
     L = _lib.load()
     with torch.cuda.device(q.device):
-        default_cap = workspace_bytes is None
-        if workspace_bytes is None:
-            # Memory the caching allocator holds but has not handed out counts
-            # as free too: the driver's free figure alone moves with every
-            # segment the allocator maps, and with it the workspace size,
-            # which then misses the cached block and allocates anew.
-            free, _ = torch.cuda.mem_get_info(q.device)
-            cached = torch.cuda.memory_reserved(q.device) - torch.cuda.memory_allocated(q.device)
-            workspace_bytes = min(BWD_WORKSPACE_CAP, (free + cached) // 4)
-        need = L.si_sparse_attn_bwd_workspace_bytes(B, S, H, D, N_kv, K, int(workspace_bytes))
-        if need < 0:
+        ws = _bwd_workspace(
+            lambda cap: L.si_sparse_attn_bwd_workspace_bytes(B, S, H, D, N_kv, K, cap), workspace_bytes, q.device)
+        if ws is None:
             raise ValueError(L.si_last_error().decode("utf-8", "replace"))
-        try:
-            ws = torch.empty((max(int(need), 16),), dtype=torch.uint8, device=q.device)
-        except torch.OutOfMemoryError:
-            if not default_cap:
-                raise
-            # The allocator's unused blocks may be split too finely to hold the
-            # workspace: size it from the driver's free memory alone.
-            free, _ = torch.cuda.mem_get_info(q.device)
-            need = L.si_sparse_attn_bwd_workspace_bytes(B, S, H, D, N_kv, K, int(min(BWD_WORKSPACE_CAP, free // 4)))
-            if need < 0:
-                raise ValueError(L.si_last_error().decode("utf-8", "replace"))
-            ws = torch.empty((max(int(need), 16),), dtype=torch.uint8, device=q.device)
         rc = L.si_sparse_attn_bwd_ragged(
             q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), attn_sink.data_ptr(),
             topk_idxs.data_ptr(), 1 if topk_idxs.dtype == torch.int64 else 0, _lib.strides(topk_idxs),
