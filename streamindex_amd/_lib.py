@@ -8,6 +8,7 @@ falls back to a CPU or torch implementation.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -117,8 +118,16 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_STRIDES = {}  # strides -> the array the library reads (it never writes one)
+
+
 def strides(t: torch.Tensor):
-    arr = (ctypes.c_int64 * t.dim())(*t.stride())
+    s = t.stride()
+    arr = _STRIDES.get(s)
+    if arr is None:
+        if len(_STRIDES) >= 4096:
+            _STRIDES.clear()
+        arr = _STRIDES[s] = (ctypes.c_int64 * len(s))(*s)
     return arr
 
 
@@ -141,6 +150,14 @@ def qkv_dtype(t: torch.Tensor) -> int:
 
 def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, free where it already is the current one."""
+    return _HERE if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def scratch(nbytes: int, device: torch.device):

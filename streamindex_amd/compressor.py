@@ -68,7 +68,7 @@ def token_compressor(
     bb = b_b.to(torch.float32).contiguous() if overlap else None
     out = torch.empty((B, n_blocks, c), dtype=c_a.dtype, device=c_a.device)
     L = _lib.load()
-    with torch.cuda.device(c_a.device):
+    with _lib.on_device(c_a.device):
         rc = L.si_token_compress(ca.data_ptr(), za.data_ptr(), ba.data_ptr(),
                                  None if cb is None else cb.data_ptr(), None if zb is None else zb.data_ptr(),
                                  None if bb is None else bb.data_ptr(), dt, B, S, c, m, int(overlap),
@@ -96,7 +96,7 @@ def softmax_gated_pool(kv: torch.Tensor, score: torch.Tensor, *, dim: int = -2) 
         return out.zero_()
     kc, sc = kv.contiguous(), score.contiguous()
     L = _lib.load()
-    with torch.cuda.device(kv.device):
+    with _lib.on_device(kv.device):
         rc = L.si_gated_pool(kc.data_ptr(), sc.data_ptr(), out.data_ptr(), dt, outer, Lk, inner,
                              _lib.stream_ptr(kv.device))
     _lib.check(rc)

@@ -62,7 +62,7 @@ def build_sliding_window_idxs(B: int, S: int, n_win: int, device) -> torch.Tenso
 def _launch_hca(out: torch.Tensor, B: int, S: int, n_win: int, n_comp: int, m_prime: int, offset: int) -> None:
     assert out.is_cuda and out.dtype == torch.int32 and out.stride(-1) == 1
     L = _lib.load()
-    with torch.cuda.device(out.device):
+    with _lib.on_device(out.device):
         rc = L.si_hca_topk_idxs(B, S, n_win, n_comp, m_prime, offset, out.data_ptr(), _lib.strides(out),
                                 _lib.stream_ptr(out.device))
     _lib.check(rc)
@@ -103,7 +103,7 @@ def csa_topk_idxs(q_idx: torch.Tensor, k_idx_compressed: torch.Tensor, indexer_w
         k8, ks = act_quant(k_idx_compressed, D_I)
         k8u = k8.view(torch.uint8)
         ks = ks[..., 0].contiguous()
-        with torch.cuda.device(q_idx.device):
+        with _lib.on_device(q_idx.device):
             rc = L.si_csa_indexer_topk_q(
                 q4.data_ptr(), _lib.strides(q4), qs.data_ptr(), _lib.strides(qs), k8u.data_ptr(), _lib.strides(k8u),
                 ks.data_ptr(), _lib.strides(ks), indexer_weights.data_ptr(),
@@ -112,7 +112,7 @@ def csa_topk_idxs(q_idx: torch.Tensor, k_idx_compressed: torch.Tensor, indexer_w
                 scores.data_ptr() if scores is not None else None, _lib.stream_ptr(q_idx.device))
         _lib.check(rc)
         return (out, scores) if return_scores else out
-    with torch.cuda.device(q_idx.device):
+    with _lib.on_device(q_idx.device):
         rc = L.si_csa_indexer_topk(
             q_idx.data_ptr(), _lib.strides(q_idx), k_idx_compressed.data_ptr(), _lib.strides(k_idx_compressed),
             indexer_weights.data_ptr(), 1 if indexer_weights.dtype == torch.bfloat16 else 0,
@@ -150,7 +150,7 @@ def build_csa_topk_idxs(indexer_scores: torch.Tensor, n_win: int, top_k: int, *,
         raise ValueError(f"n_win must be >= 0 and m > 0, got {n_win}, {m}")
     out = torch.empty((B, S, n_win + top_k), dtype=torch.int32, device=indexer_scores.device)
     L = _lib.load()
-    with torch.cuda.device(indexer_scores.device):
+    with _lib.on_device(indexer_scores.device):
         rc = L.si_csa_scores_topk(indexer_scores.data_ptr(), _lib.strides(indexer_scores), B, S, T, top_k,
                                   int(m), int(n_win), int(seq_len), out.data_ptr(), _lib.strides(out),
                                   _lib.stream_ptr(indexer_scores.device))

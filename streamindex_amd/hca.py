@@ -102,7 +102,7 @@ def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_w
     workspace fits the backward's cap, else by the general backward over the index rows."""
     B, S, H, D = q.shape
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         ws = _bwd_workspace(lambda cap: L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, n_compressed, m_prime, cap),
                             None, q.device)
         if ws is None:

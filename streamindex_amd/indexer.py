@@ -75,7 +75,7 @@ def indexer_score(q: torch.Tensor, k_idx: torch.Tensor, weights: torch.Tensor) -
     q, k_idx, weights = _prep(q, k_idx, weights)
     scores = torch.empty((B, S, T), device=q.device, dtype=torch.float32)
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         rc = L.si_indexer_score(
             q.data_ptr(), _lib.strides(q), k_idx.data_ptr(), _lib.strides(k_idx),
             weights.data_ptr(), 1 if weights.dtype == torch.bfloat16 else 0, _lib.strides(weights),
@@ -104,7 +104,7 @@ def _topk_launch(q, k_idx, weights, top_k, causal_mask, causal_ratio):
     if causal_ratio is not None and ratio <= 0:
         raise ValueError(f"causal_ratio must be a positive integer, got {causal_ratio}")
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         # Few query rows over many keys: a score scratch lets the call use the whole GPU.
         scratch, nscratch = _lib.scratch(L.si_indexer_topk_scratch_bytes(B, S, T, H_I, D_I, top_k, ratio), q.device)
         rc = L.si_indexer_topk_scratch(
@@ -270,7 +270,7 @@ def indexer_topk_q(
             causal_mask = causal_mask != 0
         mask_ptr, mask_strides = causal_mask.data_ptr(), _lib.strides(causal_mask)
     L = _lib.load()
-    with torch.cuda.device(q_fp4.device):
+    with _lib.on_device(q_fp4.device):
         rc = L.si_indexer_topk_q(
             q_fp4.data_ptr(), _lib.strides(q_fp4), q_scale.data_ptr(), _lib.strides(q_scale),
             k8.data_ptr(), _lib.strides(k8), k_scale.data_ptr(), _lib.strides(k_scale),

@@ -47,7 +47,7 @@ def _simulate(x: torch.Tensor, block_size: int, fp4: bool) -> torch.Tensor:
     xc = x.contiguous()
     y = torch.empty_like(xc)
     L = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = L.si_quant_simulate(xc.data_ptr(), y.data_ptr(), dt, xc.numel(), block_size, int(fp4),
                                  _lib.stream_ptr(x.device))
     _lib.check(rc)
@@ -81,7 +81,7 @@ def act_quant(x: torch.Tensor, block_size: int = 128, scale_fmt: Optional[str] =
     y = torch.empty(xc.shape, dtype=torch.float8_e4m3fn, device=x.device)
     s = torch.empty((*xc.shape[:-1], xc.shape[-1] // block_size), dtype=torch.float32, device=x.device)
     L = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = L.si_quant_pack(xc.data_ptr(), y.data_ptr(), s.data_ptr(), dt, xc.numel(), block_size, 0,
                              int(scale_fmt == "ue8m0"), _lib.stream_ptr(x.device))
     _lib.check(rc)
@@ -102,7 +102,7 @@ def fp4_act_quant(x: torch.Tensor, block_size: int = 32) -> Tuple[torch.Tensor, 
     y = torch.empty((*xc.shape[:-1], xc.shape[-1] // 2), dtype=torch.uint8, device=x.device)
     s = torch.empty((*xc.shape[:-1], xc.shape[-1] // block_size), dtype=torch.float32, device=x.device)
     L = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = L.si_quant_pack(xc.data_ptr(), y.data_ptr(), s.data_ptr(), dt, xc.numel(), block_size, 1, 1,
                              _lib.stream_ptr(x.device))
     _lib.check(rc)

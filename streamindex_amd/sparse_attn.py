@@ -102,7 +102,7 @@ def sparse_attn_fwd(
     o = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
     lse = torch.empty((B, S, H), dtype=torch.float32, device=q.device)
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         scratch, nscratch = _lib.scratch(L.si_sparse_attn_fwd_scratch_bytes(B, S, H, D, K), q.device)
         rc = L.si_sparse_attn_fwd_scratch(
             q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), N_kv, None, None, 0, attn_sink.data_ptr(),
@@ -161,7 +161,7 @@ def sparse_attn_fwd_kv2(
     o = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
     lse = torch.empty((B, S, H), dtype=torch.float32, device=q.device)
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         scratch, nscratch = _lib.scratch(L.si_sparse_attn_fwd_scratch_bytes(B, S, H, D, K), q.device)
         rc = L.si_sparse_attn_fwd_scratch(
             q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), N1, kv2.data_ptr(), _lib.strides(kv2),
@@ -180,12 +180,22 @@ def sparse_attn_fwd_kv2(
 # a 2 GiB workspace runs the query rows in 27 chunks (one key sort for all of
 # them) within 7 % of the time an 8 GiB one takes in 6.
 BWD_WORKSPACE_CAP = 2 << 30
+# Workspaces up to this size are taken as they are.
+BWD_SMALL_WORKSPACE = 64 << 20
 
 
 def _bwd_workspace(need, workspace_bytes: Optional[int], device: torch.device) -> Optional[torch.Tensor]:
     """A workspace of ``need(cap)`` bytes, or None where that is negative (no plan fits the cap)."""
     default_cap = workspace_bytes is None
-    if workspace_bytes is None:
+    if default_cap:
+        # A small problem's whole plan, without asking the allocator for its
+        # statistics (150 us, more than such a backward takes).
+        n = need(BWD_WORKSPACE_CAP)
+        if 0 <= n <= BWD_SMALL_WORKSPACE:
+            try:
+                return torch.empty((max(int(n), 16),), dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                pass
         # Memory the caching allocator holds but has not handed out counts
         # as free too: the driver's free figure alone moves with every
         # segment the allocator maps, and with it the workspace size,
@@ -268,7 +278,7 @@ def sparse_attn_bwd(
     dkv = torch.empty((B, N_kv, D), dtype=kv.dtype, device=q.device)
     dsink = torch.empty((H,), dtype=torch.float32, device=q.device)
     L = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         ws = _bwd_workspace(
             lambda cap: L.si_sparse_attn_bwd_workspace_bytes(B, S, H, D, N_kv, K, cap), workspace_bytes, q.device)
         if ws is None:
@@ -318,7 +328,7 @@ def build_inverted_topk(topk_idxs: torch.Tensor, n_kv: int, k_max: int, *, block
     inv_topk = torch.empty((B, n_kv, k_max), dtype=torch.int32, device=topk_idxs.device)
     inv_count = torch.empty((B, n_kv), dtype=torch.int32, device=topk_idxs.device)
     L = _lib.load()
-    with torch.cuda.device(topk_idxs.device):
+    with _lib.on_device(topk_idxs.device):
         need = L.si_build_inverted_topk_workspace_bytes(B, S, K, n_kv)
         if need < 0:
             raise ValueError(L.si_last_error().decode("utf-8", "replace"))

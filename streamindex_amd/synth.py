@@ -45,7 +45,7 @@ def device_normal(shape, dtype, *, seed: int, stream: int, scale: float = 1.0, d
         raise ValueError(f"device_normal draws bf16 or fp32, not {dtype}")
     t = torch.empty(shape, dtype=dtype, device=device)
     L = _lib.load()
-    with torch.cuda.device(t.device):
+    with _lib.on_device(t.device):
         rc = L.si_fill_normal(t.data_ptr(), 1 if dtype == torch.bfloat16 else 0, t.numel(), int(seed), int(stream),
                               float(scale), _lib.stream_ptr(t.device))
     _lib.check(rc)
