@@ -244,6 +244,12 @@ int si_hca_topk_idxs(int64_t B, int64_t S, int64_t n_win, int64_t n_compressed, 
                      int64_t idx_offset, int32_t* out_idx, const int64_t* out_strides, void* stream);
 
 /*
+ * Used columns of CSA / HCA index rows, out[s] = n_win + min(cap, (s+1)/m) for
+ * s < S (cap: picks per row), the row lengths the attention entries take.
+ */
+int si_row_len(int64_t S, int64_t n_win, int64_t cap, int64_t m, int32_t* out, void* stream);
+
+/*
  * Workspace of si_sparse_attn_bwd: the bytes needed to process the query
  * rows in the fewest chunks that fit max_bytes (one chunk when the whole
  * problem fits), or, when even one row does not fit, the one-row need.

@@ -216,6 +216,18 @@ def csa_row_len(B: int, S: int, n_win: int, top_k: int, n_compressed: int, m: in
     """``[B, S]`` int32 used columns of the fused CSA rows: the window, then
     ``min(top_k, n_compressed, (s+1)//m)`` picks (every legal key has a finite
     score, so a row holds that many); the ``-1`` rest is never run."""
-    s = torch.arange(S, device=device)
-    legal = torch.clamp((s + 1) // m, max=n_compressed)
-    return (n_win + torch.clamp(legal, max=top_k)).to(torch.int32).expand(B, S)
+    return _row_len(B, S, n_win, min(top_k, n_compressed), m, device)
+
+
+def _row_len(B: int, S: int, n_win: int, cap: int, m: int, device) -> torch.Tensor:
+    """``[B, S]`` int32 ``n_win + min(cap, (s+1)//m)`` (one kernel; on other devices torch ops)."""
+    device = torch.device(device)
+    if device.type != "cuda" or n_win < 0 or cap < 0 or m <= 0:
+        s = torch.arange(S, device=device)
+        return (n_win + torch.clamp((s + 1) // m, max=cap)).to(torch.int32).expand(B, S)
+    out = torch.empty((S,), dtype=torch.int32, device=device)
+    L = _lib.load()
+    with _lib.on_device(out.device):
+        rc = L.si_row_len(S, n_win, cap, m, out.data_ptr(), _lib.stream_ptr(out.device))
+    _lib.check(rc)
+    return out.expand(B, S)

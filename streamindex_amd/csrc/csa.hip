@@ -84,6 +84,15 @@ __global__ __launch_bounds__(256) void score_topk_kernel(ScoreTopkArgs a) {
   sel.finish(TopkRowOut{nullptr, nullptr, orow + a.n_win, a.idx_offset}, lane);
 }
 
+// Used columns of the index rows: the window, then the min(cap, (s+1)/m) legal
+// picks.  (Seven elementwise torch kernels and 14 us before.)
+__global__ __launch_bounds__(256) void row_len_kernel(int32_t* out, int S, int n_win, int cap, int m) {
+  const int s = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  if (s >= S) return;
+  const int legal = static_cast<int>((static_cast<int64_t>(s) + 1) / m);
+  out[s] = n_win + (legal < cap ? legal : cap);
+}
+
 struct HcaIdxArgs {
   int32_t* out;  // [B,S,n_win+n_comp] int32, columns contiguous
   int64_t osb, oss;
@@ -150,6 +159,18 @@ extern "C" int si_csa_scores_topk(const float* scores, const int64_t* score_stri
   if (a.top_k <= 1536) return launch_score_topk<2048>(a, st);
   if (a.top_k <= 2048) return launch_score_topk<4096>(a, st);
   return launch_score_topk<4608>(a, st);
+}
+
+extern "C" int si_row_len(int64_t S, int64_t n_win, int64_t cap, int64_t m, int32_t* out, void* stream) {
+  if (S < 0 || n_win < 0 || cap < 0 || m <= 0) return set_error(SI_ERR_INVALID, "bad dimension");
+  if (S > 0x7fffffff || m > 0x7fffffff || n_win + cap > 0x7fffffff)
+    return set_error(SI_ERR_UNSUPPORTED, "dimension exceeds int32");
+  if (S == 0) return SI_OK;
+  if (!out) return set_error(SI_ERR_INVALID, "null pointer argument");
+  hipLaunchKernelGGL(row_len_kernel, dim3(static_cast<unsigned>((S + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), out, static_cast<int>(S), static_cast<int>(n_win),
+                     static_cast<int>(cap), static_cast<int>(m));
+  return check_launch("row_len_kernel");
 }
 
 extern "C" int si_hca_topk_idxs(int64_t B, int64_t S, int64_t n_win, int64_t n_compressed, int64_t m_prime,

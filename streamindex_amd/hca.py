@@ -21,7 +21,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .csa import _launch_hca
+from .csa import _launch_hca, _row_len
 from .sparse_attn import _aligned, _bwd_workspace, sparse_attn_bwd, sparse_attn_fwd_kv2
 
 __all__ = ["flash_hca_forward", "build_hca_topk_idxs", "hca_row_len"]
@@ -126,5 +126,4 @@ def hca_row_len(B: int, S: int, n_win: int, n_compressed: int, m_prime: int, dev
     """``[B, S]`` int32 used columns of the HCA rows: the window, then the
     ``min(n_compressed, (s+1)//m_prime)`` legal compressed entries; the rest
     of each row is ``-1``, so attention never runs those tiles."""
-    s = torch.arange(S, device=device)
-    return (n_win + torch.clamp((s + 1) // m_prime, max=n_compressed)).to(torch.int32).expand(B, S)
+    return _row_len(B, S, n_win, n_compressed, m_prime, device)

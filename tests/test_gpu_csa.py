@@ -260,3 +260,15 @@ def test_csa_and_hca_backward(cuda_device):
     rows_h = build_hca_topk_idxs(B=B, seq_len=S, n_win=n_win, n_compressed=S // mp, m_prime=mp, device=q.device)
     _grad_check(lambda a, b, c, s: flash_hca_forward(a, b, c, s, n_win=n_win, m_prime=mp), q, kv, kvc_h, sink,
                 rows_h.int(), do, "hca")
+
+
+@pytest.mark.parametrize("S,n_win,cap,m", [(1, 128, 0, 4), (255, 0, 7, 1), (257, 16, 10**6, 3), (4099, 128, 512, 4)])
+def test_row_lengths(cuda_device, S, n_win, cap, m):
+    from streamindex_amd.csa import csa_row_len
+    from streamindex_amd.hca import hca_row_len
+
+    want = (n_win + torch.clamp((torch.arange(S) + 1) // m, max=cap)).to(torch.int32).expand(2, S)
+    for got in (csa_row_len(2, S, n_win, cap, cap + 5, m, "cuda"), csa_row_len(2, S, n_win, cap + 5, cap, m, "cuda"),
+                hca_row_len(2, S, n_win, cap, m, "cuda")):
+        assert got.dtype == torch.int32 and torch.equal(got.cpu(), want)
+    assert torch.equal(csa_row_len(2, S, n_win, cap, cap, m, "cpu"), want)
