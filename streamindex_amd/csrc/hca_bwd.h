@@ -2,7 +2,7 @@
 //
 // HCA's keys are not scattered: query s attends to the window s-n_win+1 .. s
 // and to every compressed entry i < (s+1)/m.  The general backward writes one
-// dkv row per (query, slot) and sorts and sums them by key; here 64 keys and a
+// dkv row per (query, slot) and sorts and sums them by key; here 128 keys and a
 // block of consecutive queries meet in one workgroup, which sums their dkv in
 // MFMA accumulators, so nothing is written per pair:
 //   1. hca_bwd_idx_kernel: index rows whose window part starts at a multiple of
@@ -10,21 +10,22 @@
 //      (s-n_win+1)/32 + i whatever s is.
 //   2. sparse_attn_bwd_rows_kernel on those rows: dq, dsink terms, and P / dS of
 //      every tile (8 KiB each) in its register layout.
-//   3. hca_bwd_dkv_kernel: per (64 keys, RB query rows) the sum over the rows'
+//   3. hca_bwd_dkv_kernel: per (128 keys, RB query rows) the sum over the rows'
 //      heads of dS q + P dO, fp32, to a partial buffer.
 //   4. hca_bwd_reduce_kernel: each key's partials in block order.
 // Every sum has a fixed order, so repeated calls are bit-identical.
 //
-// Bound: step 2 (its gathers and coefficients) and step 3's copies: a row's Q
-// and dO come through LDS once per 64-key group it meets (4 to 5 at S = 16K),
-// 32 heads at a time so that the next half is copied while one is multiplied.
-// Measured at S = 16,384, 64 heads, D = 576, n_win = m = 128: rows 1.80,
-// dkv 1.55, reduction 0.07 ms, against 1.76 + 1.45 + 1.26 + 0.11 ms (rows, dkv
-// rows, reduction, sort) of the general backward over 3.2M pairs; forward and
-// backward 5.51 -> 4.4 ms.
+// Bound: step 2 (its gathers and coefficients) and step 3's chain per row (see
+// its comment).  Measured at S = 16,384, 64 heads, D = 576, n_win = m = 128: rows
+// 1.80, dkv 1.41, reduction 0.07 ms, against 1.76 + 1.45 + 1.26 + 0.11 ms (rows,
+// dkv rows, reduction, sort) of the general backward over 3.2M pairs; forward
+// and backward 5.51 -> 4.2 ms.
 #pragma once
 
 namespace si {
+
+constexpr int kHcaShift = 7;  // 128 keys (four 32-key tiles) per group
+constexpr int kHcaKeys = 1 << kHcaShift;
 
 struct HcaBwdArgs {
   int n_win, m, T;
@@ -32,16 +33,18 @@ struct HcaBwdArgs {
   int RB;          // query rows of a block (a multiple of 32)
   int b0, nb;      // batches of this chunk
   int s0, s1;      // query rows of this chunk (s0 a multiple of RB)
-  int GW, ncg;     // window / compressed 64-key groups of a block
-  float* part;     // [nb, blocks, GW + ncg, 64, D]
+  int GW, ncg;     // window / compressed key groups of a block
+  float* part;     // [nb, blocks, GW + ncg, kHcaKeys, D]
   float* acc;      // [B, N, D] fp32 sums of the earlier chunks
   uint16_t* dkv;   // [B, N, D]
   int64_t dsb, dsn;
   int first, last;  // first / last chunk of the batch
 };
 
-// First 64-key window group that row block blk touches (keys below 0 count).
-__device__ __forceinline__ int hca_group_lo(const HcaBwdArgs& h, int blk) { return (blk * h.RB - h.n_win + 1) >> 6; }
+// First window group that row block blk meets (keys below 0 count).
+__device__ __forceinline__ int hca_group_lo(const HcaBwdArgs& h, int blk) {
+  return (blk * h.RB - h.n_win + 1) >> kHcaShift;
+}
 
 // Query rows of (block, group j): the block's rows inside the chunk that have a
 // key of the group.
@@ -50,12 +53,12 @@ __device__ __forceinline__ void hca_item_rows(const HcaBwdArgs& h, int blk, int 
   r1 = (blk + 1) * h.RB < h.s1 ? (blk + 1) * h.RB : h.s1;
   if (j < h.GW) {
     const int kg = hca_group_lo(h, blk) + j;
-    const int lo = 64 * kg, hi = 64 * kg + 63 + h.n_win;  // rows lo .. hi-1 see keys 64 kg .. 64 kg + 63
+    const int lo = kHcaKeys * kg, hi = lo + kHcaKeys - 1 + h.n_win;  // rows lo .. hi-1 see the group's keys
     if (kg < 0) r1 = r0;
     r0 = r0 > lo ? r0 : lo;
     r1 = r1 < hi ? r1 : hi;
   } else {
-    const int64_t lo = static_cast<int64_t>(h.m) * (64 * (j - h.GW) + 1) - 1;
+    const int64_t lo = static_cast<int64_t>(h.m) * (kHcaKeys * (j - h.GW) + 1) - 1;
     if (r0 < lo) r0 = lo < r1 ? static_cast<int>(lo) : r1;
   }
 }
@@ -89,10 +92,10 @@ struct HcaDkvShape {
   static constexpr int CPR = D / 8;
   static constexpr int CPP = CPR + 2;          // chunks per LDS row: padded as in DkvShape (conflict-free transposing reads)
   static constexpr int QROW = CPP * 16;
-  static constexpr int HALF = 32 * QROW;       // 32 heads of Q or of dO
-  static constexpr int BUF = 2 * HALF;         // Q then dO
+  static constexpr int PART = 16 * QROW;       // 16 heads of Q or of dO
+  static constexpr int BUF = 2 * PART;         // Q then dO
   static constexpr int NW = 8;                      // waves, two per SIMD
-  static constexpr int COPIES = 2 * 32 * CPP / 64;  // 64-lane copies of a stage
+  static constexpr int COPIES = 2 * 16 * CPP / 64;  // 64-lane copies of a stage (CPP is even)
   static constexpr int CPW = (COPIES + NW - 1) / NW;  // copies per wave
   // 16-dimension blocks: MBW each for waves 0..3, the rest in equal shares for
   // waves 4..7, so that the two waves of a SIMD hold MBT / 4 together.
@@ -100,11 +103,11 @@ struct HcaDkvShape {
   static constexpr int MBW = (MBT + 7) / 8;
   static constexpr int MBW2 = MBT > 4 * MBW ? (MBT - 4 * MBW) / 4 : 0;
   static_assert(MBT <= 4 * MBW || (MBT - 4 * MBW) % 4 == 0, "blocks of waves 4..7");
-  // Coefficients: [tile][P, dS][producer wave][4-key group][head][16 bytes], the
-  // key groups 320 bytes apart (256 would put a transposing read's four in one bank)
+  // Coefficients: [tile][P, dS][4-key group][head][16 bytes], the key groups 320
+  // bytes apart (256 would put a transposing read's four in one bank)
   static constexpr int CG = 320;
   static constexpr int CW4 = 4 * CG;
-  static constexpr int COEF = 2 * 2 * 2 * CW4;
+  static constexpr int COEF = 4 * 2 * CW4;
 };
 
 // 16 bytes per lane from memory to LDS (64 lanes: consecutive slots from dst).
@@ -112,13 +115,16 @@ __device__ __forceinline__ void hca_copy16(const uint16_t* src, char* dst) {
   __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 16, 0, 0);
 }
 
-// dkv^T [D x 64 keys] += [Q^T | dO^T] [D x 64] . [dS; P] [64 x 64 keys] per stage
-// (one query row, 32 heads), the operands as in sparse_attn_bwd_dkv_rows_kernel.
-// Two waves per SIMD: one's copies, waits and fragment reads run beside the
-// other's MFMAs.  Bound: the copies, 16 bytes a clock and CU (8.7 TB/s from the
-// L2; the same rows from L2 throughout take as long, without the copies the
-// kernel takes 0.83 instead of 1.55 ms; spreading them over the blocks, or
-// touching the lines two rows ahead, changed nothing).
+// dkv^T [D x 128 keys] += [Q^T | dO^T] [D x 32] . [dS; P] [32 x 128 keys] per
+// stage: one query row, 16 heads, whose dS against Q and P against dO make one
+// 32-deep MFMA step.  The operands are read as in
+// sparse_attn_bwd_dkv_rows_kernel.  Two waves per SIMD: one's copies, waits and
+// fragment reads run beside the other's MFMAs.  128 keys per group: a row is
+// copied and read 3 times at S = 16K (4.5 times with 64 keys and 32-head stages:
+// 1.55 ms, this 1.41).  A stage takes 3,900 clocks for 1,152 of MFMA per SIMD:
+// the copies, the fragment reads behind the barrier and the MFMAs follow one
+// another.  Two more stages in flight (a ring of four) measured 1.39, touching
+// the lines two rows ahead or spreading the copies over the blocks nothing.
 template <int D, bool F16>
 __global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdArgs h) {
   using HS = HcaDkvShape<D>;
@@ -142,44 +148,40 @@ __global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdA
   hca_item_rows(h, blk, j, r0, r1);
   if (r0 >= r1) return;
   const bool window = j < h.GW;
-  const int kt = 2 * (window ? hca_group_lo(h, blk) + j : j - h.GW);  // first 32-key tile of the group
+  const int kt = 4 * (window ? hca_group_lo(h, blk) + j : j - h.GW);  // first 32-key tile of the group
   const int blk_lo = wave < 4 ? wave * MBW : 4 * MBW + (wave - 4) * HS::MBW2;  // this wave's dimension blocks
 
   // Copies of a stage: LDS chunk e (16 bytes) is chunk e % CPP of head
-  // (e / CPP) % 32 of Q (e < 32 CPP) or dO; the pad chunks re-read chunk 0.
-  // Copy n = NW i + wave is wholly one of the two (32 CPP is a multiple of 64).
+  // (e / CPP) % 16 of Q (e < 16 CPP) or dO; the pad chunks re-read chunk 0.
   int voff[HS::CPW];  // byte offset from the stage's first head
 #pragma unroll
   for (int i = 0; i < HS::CPW; ++i) {
     const int n = i * HS::NW + wave;
     const int e = n * 64 + lane;
     const int c = e % HS::CPP;
-    voff[i] = static_cast<int>(((e / HS::CPP) % 32) * (n < HS::COPIES / 2 ? a.qsh : a.gsh) + (c < HS::CPR ? c : 0) * 8) * 2;
+    voff[i] = static_cast<int>(((e / HS::CPP) % 16) * (e < 16 * HS::CPP ? a.qsh : a.gsh) + (c < HS::CPR ? c : 0) * 8) * 2;
   }
+  const int nq = (a.H + 15) / 16;  // 16-head parts of a row
   struct Stage {
-    int s, hg, half;
+    int s, part;
   };
-  auto next = [&](Stage x) {
-    if (x.half == 0) return Stage{x.s, x.hg, 1};
-    return x.hg + 1 < a.HG ? Stage{x.s, x.hg + 1, 0} : Stage{x.s + 1, 0, 0};
-  };
+  auto next = [&](Stage x) { return x.part + 1 < nq ? Stage{x.s, x.part + 1} : Stage{x.s + 1, 0}; };
   auto copy_stage = [&](const Stage& x, int buf) {
-    const int h0 = x.hg * 64 + x.half * 32;
+    const int h0 = x.part * 16;
     const char* qs = reinterpret_cast<const char*>(a.q + b * a.qsb + static_cast<int64_t>(x.s) * a.qss + h0 * a.qsh);
     const char* gs = reinterpret_cast<const char*>(a.dout + b * a.gsb + static_cast<int64_t>(x.s) * a.gss + h0 * a.gsh);
     char* dst = qd_lds + buf * HS::BUF;
-    const bool whole = h0 + 32 <= a.H;
+    const bool whole = h0 + 16 <= a.H;
 #pragma unroll
     for (int i = 0; i < HS::CPW; ++i) {
       const int n = i * HS::NW + wave;
       if (n < HS::COPIES) {
-        const bool isq = n < HS::COPIES / 2;
+        const int e = n * 64 + lane;
+        const bool isq = e < 16 * HS::CPP;
         int off = voff[i];
         if (!whole) {
-          // heads past H re-read the last one below it, or head H-1 (their P and
-          // dS are 0): step back whole heads
-          const int e = n * 64 + lane;
-          const int hd = (e / HS::CPP) % 32;
+          // heads past H re-read head H-1 (their P and dS are 0)
+          const int hd = (e / HS::CPP) % 16;
           const int over = h0 + hd - (a.H - 1);
           if (over > 0) off -= over * static_cast<int>(isq ? a.qsh : a.gsh) * 2;
         }
@@ -187,56 +189,51 @@ __global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdA
       }
     }
   };
-  // Coefficients of a stage: tiles kt and kt+1, 32 heads (two producer waves),
-  // by waves 0..3; zero where the query row has no such tile.
+  // Coefficients of a stage: tiles kt .. kt+3, 16 heads (one producer wave), 16
+  // bytes a thread: wave 2 k + 0 / 1 takes P / dS of tile kt + k; zero where the
+  // query row has no such tile.
   const int64_t nr = h.s1 - h.s0;
-  u32x4 cf[2];
+  u32x4 cf;
   auto load_coef = [&](const Stage& x) {
-    if (wave >= 4) return;
     const int64_t lrow = (b - h.b0) * nr + (x.s - h.s0);
-    const uint16_t* row = a.coef + (lrow * a.HG + x.hg) * a.ntiles * kCoefTile;
-    const int t = threadIdx.x;  // [P, dS][producer wave][lane]
-    const int off = ((t >> 7) * 4 + 2 * x.half + ((t >> 6) & 1)) * 512 + (t & 63) * 8;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      int ti = kt + k;
-      bool ok;
-      if (window) {
-        ti -= (x.s - h.n_win + 1) >> 5;
-        ok = ti >= 0 && ti < h.wtiles;
-      } else {
-        ok = static_cast<int64_t>(h.m) * (ti * 32 + 1) <= x.s + 1 && ti * 32 < h.T;  // its first entry is legal
-        ti += h.wtiles;
-      }
-      cf[k] = ok ? *reinterpret_cast<const u32x4*>(row + static_cast<int64_t>(ti) * kCoefTile + off) : u32x4{0u, 0u, 0u, 0u};
+    const uint16_t* row = a.coef + (lrow * a.HG + (x.part >> 2)) * a.ntiles * kCoefTile;
+    int ti = kt + (wave >> 1);
+    bool ok;
+    if (window) {
+      ti -= (x.s - h.n_win + 1) >> 5;
+      ok = ti >= 0 && ti < h.wtiles;
+    } else {
+      ok = static_cast<int64_t>(h.m) * (ti * 32 + 1) <= x.s + 1 && ti * 32 < h.T;  // its first entry is legal
+      ti += h.wtiles;
     }
+    const int off = ((wave & 1) * 4 + (x.part & 3)) * 512 + lane * 8;
+    cf = ok ? *reinterpret_cast<const u32x4*>(row + static_cast<int64_t>(ti) * kCoefTile + off) : u32x4{0u, 0u, 0u, 0u};
   };
+  char* const cst = coef_lds + wave * HS::CW4 + (lane >> 4) * HS::CG + (lane & 15) * 16;  // where they go
 
-  const uint32_t qd0 = lds_addr(qd_lds) + (8 * g + (i16 >> 2)) * HS::QROW + 8 * (i16 & 3) + blk_lo * 32;
-  const int bh = 8 * g + (i16 >> 2);  // head of the 32
-  const uint32_t cf0 = lds_addr(coef_lds) + (bh >> 4) * HS::CW4 + (i16 & 3) * HS::CG + (bh & 15) * 16;
-  const int cst = ((threadIdx.x >> 6) & 3) * HS::CW4 + (lane >> 4) * HS::CG + (lane & 15) * 16;  // where load_coef's words go
+  // k of the MFMA step: 0..15 the 16 heads of Q / dS, 16..31 those of dO / P.  Lane
+  // group g holds k = 8 g .. 8 g + 7: heads 8 (g & 1) .. of the first or second.
+  const int kh = 8 * (g & 1) + (i16 >> 2);
+  const uint32_t qd0 = lds_addr(qd_lds) + (g >> 1) * HS::PART + kh * HS::QROW + 8 * (i16 & 3) + blk_lo * 32;
+  const uint32_t cf0 = lds_addr(coef_lds) + (g < 2 ? HS::CW4 : 0) + (i16 & 3) * HS::CG + kh * 16;
 
   // The stages with NB dimension blocks (a compile-time count: LDS reads in
   // flight must not cross control flow, where their registers could be copied
   // before the data lands).
   auto stages = [&](auto NBC) {
     constexpr int NB = decltype(NBC)::value;
-    f32x4 acc[NB > 0 ? NB : 1][4];
+    f32x4 acc[NB > 0 ? NB : 1][8];
 #pragma unroll
     for (int m = 0; m < NB; ++m)
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Stage cur{r0, 0, 0};
+      for (int nb = 0; nb < 8; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Stage cur{r0, 0};
     copy_stage(cur, 0);
     load_coef(cur);
     int buf = 0;
     for (; cur.s < r1; buf ^= 1) {
       __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));  // this stage's copies and coefficients landed (issued a stage ago)
-      if (wave < 4) {
-        *reinterpret_cast<u32x4*>(coef_lds + cst) = cf[0];
-        *reinterpret_cast<u32x4*>(coef_lds + 4 * HS::CW4 + cst) = cf[1];
-      }
+      *reinterpret_cast<u32x4*>(cst) = cf;
       attn_tile_barrier();
       // (the other buffer was last read in the previous stage, which every wave has left)
       cur = next(cur);
@@ -245,74 +242,59 @@ __global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdA
         load_coef(cur);
       }
       if constexpr (NB > 0) {
-        // k-step 0: dS of the 32 heads against Q; 1: P against dO.  Key blocks
-        // nb: 16 (nb & 1) of tile nb >> 1.
-        v4i16 blo[2][4], bhi[2][4];
-        attn_static_for<0, 2>([&](auto KC) {
-          attn_static_for<0, 4>([&](auto NC) {
-            constexpr int ks = decltype(KC)::value;
-            constexpr int nb = decltype(NC)::value;
-            constexpr int off = (nb >> 1) * 4 * HS::CW4 + (ks == 0 ? 2 * HS::CW4 : 0) + 8 * (nb & 1);
-            blo[ks][nb] = tr_read<off>(cf0);
-            bhi[ks][nb] = tr_read<off + 64>(cf0);
-          });
+        // Key blocks nb: 16 (nb & 1) of tile nb >> 1.
+        v4i16 blo[8], bhi[8];
+        attn_static_for<0, 8>([&](auto NC) {
+          constexpr int nb = decltype(NC)::value;
+          constexpr int off = (nb >> 1) * 2 * HS::CW4 + 8 * (nb & 1);
+          blo[nb] = tr_read<off>(cf0);
+          bhi[nb] = tr_read<off + 64>(cf0);
         });
         const uint32_t qa = qd0 + buf * HS::BUF;
-        v4i16 alo[2][2], ahi[2][2];
+        v4i16 alo[2], ahi[2];
         auto a_read = [&](auto JC) {
           constexpr int m = decltype(JC)::value;
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            alo[m & 1][ks] = tr_read<m * 32>(qa + ks * HS::HALF);
-            ahi[m & 1][ks] = tr_read<m * 32 + 4 * HS::QROW>(qa + ks * HS::HALF);
-          }
+          alo[m & 1] = tr_read<m * 32>(qa);
+          ahi[m & 1] = tr_read<m * 32 + 4 * HS::QROW>(qa);
         };
         a_read(std::integral_constant<int, 0>{});
-        lds_wait_n<4>();
-        bf16x8 bfr[2][4];
+        lds_wait_n<2>();
+        bf16x8 bfr[8];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-          for (int nb = 0; nb < 4; ++nb) {
-            reg_tie(blo[ks][nb]);
-            reg_tie(bhi[ks][nb]);
-            bfr[ks][nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[ks][nb], bhi[ks][nb], 0, 1, 2, 3, 4, 5, 6, 7));
-          }
+        for (int nb = 0; nb < 8; ++nb) {
+          reg_tie(blo[nb]);
+          reg_tie(bhi[nb]);
+          bfr[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[nb], bhi[nb], 0, 1, 2, 3, 4, 5, 6, 7));
+        }
         attn_static_for<0, NB>([&](auto JC) {
           constexpr int m = decltype(JC)::value;
           if constexpr (m + 1 < NB) {
             a_read(std::integral_constant<int, m + 1>{});
-            lds_wait_n<4>();
+            lds_wait_n<2>();
           } else {
             lds_wait_n<0>();
           }
+          reg_tie(alo[m & 1]);
+          reg_tie(ahi[m & 1]);
+          const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo[m & 1], ahi[m & 1], 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            reg_tie(alo[m & 1][ks]);
-            reg_tie(ahi[m & 1][ks]);
-          }
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo[m & 1][ks], ahi[m & 1][ks], 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) acc[m][nb] = mfma16x16x32<F16>(af, bfr[ks][nb], acc[m][nb]);
-          }
+          for (int nb = 0; nb < 8; ++nb) acc[m][nb] = mfma16x16x32<F16>(af, bfr[nb], acc[m][nb]);
         });
       }
       attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
     }
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
-      mfma_result_fence(acc[m][0], acc[m][1]);
-      mfma_result_fence(acc[m][2], acc[m][3]);
+#pragma unroll
+      for (int nb = 0; nb < 8; nb += 2) mfma_result_fence(acc[m][nb], acc[m][nb + 1]);
     }
     // lane (key 16 nb + i16 of the group, g) holds dimensions 16 mbi + 4 g + 0..3
-    float* out = h.part + static_cast<int64_t>(item) * 64 * D;
+    float* out = h.part + static_cast<int64_t>(item) * kHcaKeys * D;
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
       if (blk_lo + m < HS::MBT) {  // (at D = 32 waves 2 and 3 hold no block of the row)
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
+        for (int nb = 0; nb < 8; ++nb)
           *reinterpret_cast<f32x4*>(out + (nb * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = acc[m][nb];
       }
     }
@@ -333,9 +315,9 @@ __global__ __launch_bounds__(256) void hca_bwd_reduce_kernel(HcaBwdArgs h, int S
   const int blk0 = h.s0 / h.RB;
   const int nblk = (h.s1 + h.RB - 1) / h.RB - blk0;
   const bool window = n < S;
-  const int grp = (window ? n : n - S) >> 6;
-  const int64_t lo = window ? 64 * grp : static_cast<int64_t>(h.m) * (64 * grp + 1) - 1;
-  const int64_t hi = window ? 64 * grp + 63 + h.n_win : h.s1;
+  const int grp = (window ? n : n - S) >> kHcaShift;
+  const int64_t lo = window ? kHcaKeys * grp : static_cast<int64_t>(h.m) * (kHcaKeys * grp + 1) - 1;
+  const int64_t hi = window ? lo + kHcaKeys - 1 + h.n_win : h.s1;
   int64_t from = lo > h.s0 ? lo : h.s0, to = hi < h.s1 ? hi : h.s1;  // rows with a key of the group
   if (window ? h.GW == 0 : grp >= h.ncg) to = from;
   if (from >= to && !h.first && !h.last) return;
@@ -348,7 +330,7 @@ __global__ __launch_bounds__(256) void hca_bwd_reduce_kernel(HcaBwdArgs h, int S
     auto part = [&](int q) {
       const int j = window ? grp - hca_group_lo(h, q) : h.GW + grp;
       const int64_t item = (static_cast<int64_t>(b - h.b0) * nblk + (q - blk0)) * per + j;
-      return *reinterpret_cast<const f32x4*>(h.part + (item * 64 + ((window ? n : n - S) & 63)) * D + d);
+      return *reinterpret_cast<const f32x4*>(h.part + (item * kHcaKeys + ((window ? n : n - S) & (kHcaKeys - 1))) * D + d);
     };
     for (int q = q0; q <= q1; q += 8) {
       f32x4 v[8];
@@ -386,8 +368,8 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   p->RB = RB;
   p->wtiles = n_win > 0 ? static_cast<int>((n_win + 31 + 31) / 32) : 0;
   p->ntiles = p->wtiles + static_cast<int>((T + 31) / 32);
-  p->GW = n_win > 0 ? static_cast<int>((RB + n_win - 2) / 64 + 2) : 0;
-  p->ncg = static_cast<int>((T + 63) / 64);
+  p->GW = n_win > 0 ? static_cast<int>((RB + n_win - 2) / kHcaKeys + 2) : 0;
+  p->ncg = static_cast<int>((T + kHcaKeys - 1) / kHcaKeys);
   size_t off = 0;
   auto take = [&](int64_t bytes) {
     const size_t at = off;
@@ -400,7 +382,7 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   p->idx = take(S * (32 * p->wtiles + T) * 4);
   p->row_len = take(S * 4);
   p->coef = take(nb * rows * HG * p->ntiles * kCoefTile * 2);
-  p->part = take(nb * blocks * (p->GW + p->ncg) * 64 * D * 4);
+  p->part = take(nb * blocks * (p->GW + p->ncg) * kHcaKeys * D * 4);
   p->total = off;
 }
 
@@ -409,7 +391,7 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
 static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, size_t bytes, HcaPlan* p) {
   for (int RB = 64; RB >= 32; RB /= 2) {
     hca_plan_for(B, S, H, D, n_win, T, RB, S, B, p);
-    if (RB == 32 || B * ((S + RB - 1) / RB) * (p->GW + p->ncg) >= 1024) break;
+    if (RB == 32 || B * ((S + RB - 1) / RB) * (p->GW + p->ncg) >= 512) break;
   }
   if (p->total <= bytes) return true;
   const int RB = p->RB;

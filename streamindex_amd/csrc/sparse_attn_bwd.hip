@@ -1172,7 +1172,7 @@ static int hca_check(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, 
   const int64_t lim = int64_t{1} << 30;
   const int64_t HG = (H + 63) / 64;
   if (S >= lim || n_win >= lim || T >= lim || m >= lim || H >= lim || B * (S + T) >= lim || B * S * HG >= lim ||
-      S * (n_win + T + 64) >= (int64_t{1} << 40) || n_win + T == 0 || m * (T + 64) >= (int64_t{1} << 40))
+      S * (n_win + T + 64) >= (int64_t{1} << 40) || n_win + T == 0 || m * (T + 128) >= (int64_t{1} << 40))
     return set_error(SI_ERR_UNSUPPORTED, "HCA backward: shape outside the aligned path");
   return SI_OK;
 }
