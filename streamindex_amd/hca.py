@@ -10,7 +10,7 @@ arange/where/cat passes.
 
 ``use_triton`` is accepted for compatibility and selects nothing (one HIP
 implementation).  The backward knows the rows' structure too: it sums dkv for
-64 keys and a block of queries at a time (``si_hca_attn_bwd``) instead of
+128 keys and a block of queries at a time (``si_hca_attn_bwd``) instead of
 sorting (query, slot) pairs by key.
 """
 
