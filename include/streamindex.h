@@ -302,8 +302,9 @@ int si_sparse_attn_bwd_ragged(const void* q, const int64_t* q_strides, const voi
  * Backward of the HCA composition (flash_sparse/hca.py:54-95): the gradients
  * si_sparse_attn_bwd_ragged gives for the index rows si_hca_topk_idxs builds
  * (n_win window columns, then every entry i < (s+1)/m of the T compressed ones
- * at S + i), for kv = [B, S + T, D] = [kv ; kv_compressed], without index rows,
- * a sort or per-slot dkv rows.  workspace: at least
+ * at S + i), for kv = [B, N_kv, D] = [kv ; kv_compressed], without index rows,
+ * a sort or per-slot dkv rows.  N_kv must be S + T, one kv row per query (the
+ * general entry serves other lengths).  workspace: at least
  * si_hca_attn_bwd_workspace_bytes(..., max_bytes) bytes, -1 for a shape or a
  * max_bytes it does not serve (the general entry then does).  Every dimension
  * is positive except T and n_win, not both of which are 0.
@@ -313,9 +314,9 @@ int64_t si_hca_attn_bwd_workspace_bytes(int64_t B, int64_t S, int64_t H, int64_t
 int si_hca_attn_bwd(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,
                     const float* attn_sink, const void* o, const int64_t* o_strides, const float* lse,
                     const int64_t* lse_strides, const void* dout, const int64_t* do_strides, int64_t B, int64_t S,
-                    int64_t H, int64_t D, int64_t n_win, int64_t T, int64_t m, float softmax_scale, int qkv_dtype,
-                    void* dq, const int64_t* dq_strides, void* dkv, const int64_t* dkv_strides, float* dsink,
-                    void* workspace, int64_t workspace_bytes, void* stream);
+                    int64_t H, int64_t D, int64_t N_kv, int64_t n_win, int64_t T, int64_t m, float softmax_scale,
+                    int qkv_dtype, void* dq, const int64_t* dq_strides, void* dkv, const int64_t* dkv_strides,
+                    float* dsink, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * si_sparse_attn_bwd_ragged without allocation: the workspace is a

@@ -1201,12 +1201,14 @@ extern "C" int64_t si_hca_attn_bwd_workspace_bytes(int64_t B, int64_t S, int64_t
 extern "C" int si_hca_attn_bwd(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,
                                const float* attn_sink, const void* o, const int64_t* o_strides, const float* lse,
                                const int64_t* lse_strides, const void* dout, const int64_t* do_strides, int64_t B,
-                               int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, int64_t m,
+                               int64_t S, int64_t H, int64_t D, int64_t N_kv, int64_t n_win, int64_t T, int64_t m,
                                float softmax_scale, int qkv_dtype, void* dq, const int64_t* dq_strides, void* dkv,
                                const int64_t* dkv_strides, float* dsink, void* workspace, int64_t workspace_bytes,
                                void* stream) {
   int rc = hca_check(B, S, H, D, n_win, T, m);
   if (rc) return rc;
+  // (the kernels read and write kv and dkv rows 0 .. S + T - 1)
+  if (N_kv != S + T) return set_error(SI_ERR_INVALID, "N_kv must be S + T");
   if (qkv_dtype != SI_DTYPE_BF16 && qkv_dtype != SI_DTYPE_F16)
     return set_error(SI_ERR_INVALID, "qkv_dtype must be SI_DTYPE_BF16 (0) or SI_DTYPE_F16 (1)");
   if (!q_strides || !kv_strides || !o_strides || !lse_strides || !do_strides || !dq_strides || !dkv_strides)

@@ -98,13 +98,16 @@ class _HcaAttnFunc(torch.autograd.Function):
 
 
 def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_win, m_prime):
-    """``(dq, dkv, dsink)`` for ``kv = [kv ; kv_compressed]``, by ``si_hca_attn_bwd`` where it serves the shape and its
-    workspace fits the backward's cap, else by the general backward over the index rows."""
+    """``(dq, dkv, dsink)`` for ``kv = [kv ; kv_compressed]``, by ``si_hca_attn_bwd`` where it serves the shape (one kv row
+    per query) and its workspace fits the backward's cap, else by the general backward over the index rows."""
     B, S, H, D = q.shape
+    N_kv = kv.shape[1]
     L = _lib.load()
     with _lib.on_device(q.device):
-        ws = _bwd_workspace(lambda cap: L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, n_compressed, m_prime, cap),
-                            None, q.device)
+        ws = None
+        if N_kv == S + n_compressed:
+            ws = _bwd_workspace(
+                lambda cap: L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, n_compressed, m_prime, cap), None, q.device)
         if ws is None:
             topk_idxs, row_len = _rows(B, S, n_win, n_compressed, m_prime, q.device)
             return sparse_attn_bwd(q, kv, attn_sink, topk_idxs, o, lse, do, softmax_scale, row_len=row_len)
@@ -114,8 +117,8 @@ def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_w
         dsink = torch.empty((H,), dtype=torch.float32, device=q.device)
         rc = L.si_hca_attn_bwd(
             q.data_ptr(), _lib.strides(q), kv.data_ptr(), _lib.strides(kv), attn_sink.data_ptr(), o.data_ptr(),
-            _lib.strides(o), lse.data_ptr(), _lib.strides(lse), do.data_ptr(), _lib.strides(do), B, S, H, D, n_win,
-            n_compressed, m_prime, float(D ** -0.5 if softmax_scale is None else softmax_scale), _lib.qkv_dtype(q),
+            _lib.strides(o), lse.data_ptr(), _lib.strides(lse), do.data_ptr(), _lib.strides(do), B, S, H, D, N_kv,
+            n_win, n_compressed, m_prime, float(D ** -0.5 if softmax_scale is None else softmax_scale), _lib.qkv_dtype(q),
             dq.data_ptr(), _lib.strides(dq), dkv.data_ptr(), _lib.strides(dkv), dsink.data_ptr(), ws.data_ptr(),
             ws.numel(), _lib.stream_ptr(q.device))
     _lib.check(rc)

@@ -116,3 +116,17 @@ def test_oracle(cuda_device):
     for x, y in ((dq[0], rdq), (dkv[0], rdkv[:S]), (dkvc[0], rdkv[S:])):
         assert np.linalg.norm(x.float().cpu().numpy() - y) <= 1e-2 * np.linalg.norm(y)
     assert np.abs(ds.cpu().numpy() - rds).max() <= 1e-3 * max(1.0, np.abs(rds).max())
+
+
+@pytest.mark.parametrize("n1", [60, 99, 101, 150])
+def test_kv_of_another_length(cuda_device, n1):
+    # (the general backward serves these: the aligned kernels assume a kv row per query)
+    B, S, H, D, T, n_win, m = 2, 100, 16, 64, 12, 24, 8
+    q, _, kvc, sink, do = _inputs(B, S, H, D, T, torch.bfloat16, n1)
+    kv = synth.csa_attn_inputs(B, n1, H, D, T, seed=n1, scale=0.7)[1]
+    got = _grads(q, kv, kvc, sink, do, n_win, m)
+    rows, row_len = hca._rows(B, S, n_win, T, m, q.device)
+    full = torch.cat([kv, kvc], 1)
+    o, lse = sparse_attn_fwd(q, full, sink, rows, row_len=row_len)
+    dq, dkv, ds = sparse_attn_bwd(q, full, sink, rows, o, lse, do, row_len=row_len)
+    _check(got, (dq, dkv[:, :n1], dkv[:, n1:], ds), 0.0, f"{n1} kv rows")

@@ -1,0 +1,74 @@
+"""Host side of the HCA backward (no kernel is launched): which calls take
+si_hca_attn_bwd, and what that entry refuses.
+
+si_hca_attn_bwd reads and writes rows 0 .. S + T - 1 of [kv ; kv_compressed],
+so it serves calls with one kv row per query only; the forward takes any number
+of kv rows (indices past them are masked), and so does the general backward.
+"""
+
+from __future__ import annotations
+
+import contextlib
+import ctypes
+import os
+
+import pytest
+import torch
+
+from streamindex_amd import _lib, hca
+from streamindex_amd.build import LIB_PATH
+
+
+class _Refused(Exception):
+    pass
+
+
+@pytest.mark.parametrize("n1", [1, 7, 9, 40])
+def test_other_kv_lengths_take_the_general_backward(monkeypatch, n1):
+    S, H, D, T = 8, 2, 32, 3
+
+    class Lib:
+        def si_hca_attn_bwd_workspace_bytes(self, *a):
+            raise _Refused
+
+    general = []
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    monkeypatch.setattr(_lib, "on_device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(hca, "_rows", lambda *a: ("rows", "row_len"))
+    monkeypatch.setattr(hca, "sparse_attn_bwd", lambda *a, **k: general.append((a, k)) or (1, 2, 3))
+
+    def call(n):
+        q = torch.zeros(1, S, H, D)
+        kv = torch.zeros(1, n + T, D)
+        return hca._hca_attn_bwd(q, kv, torch.zeros(H), q, torch.zeros(1, S, H), q, T, None, 4, 2)
+
+    assert call(n1) == (1, 2, 3)
+    (a, k), = general
+    assert a[1].shape[1] == n1 + T and a[3] == "rows" and k["row_len"] == "row_len"
+    with pytest.raises(_Refused):
+        call(S)
+
+
+def _entry(B, S, H, D, N, n_win, T, m, hs=None):
+    if not os.path.exists(LIB_PATH):
+        pytest.skip("libstreamindex.so not built (run __graft_entry__.build())")
+    lib = _lib.load()
+    i64 = lambda *v: (ctypes.c_int64 * len(v))(*v)  # noqa: E731
+    hs = D if hs is None else hs
+    q4 = i64(S * H * D, H * D, hs, 1)
+    fake = 0x1000  # never dereferenced: every call below fails validation
+    kv = i64(N * D, D, 1)
+    rc = lib.si_hca_attn_bwd(fake, q4, fake, kv, fake, fake, q4, fake, i64(S * H, H, 1), fake, q4, B, S, H, D, N, n_win, T,
+                             m, 0.1, 0, fake, q4, fake, kv, fake, fake, 0, None)
+    return rc, lib.si_last_error().decode()
+
+
+@pytest.mark.parametrize("N", [0, 1, 66, 68, 200])
+def test_entry_refuses_other_row_counts(N):
+    rc, msg = _entry(1, 64, 16, 64, N, 16, 3, 16)
+    assert rc == _lib.SI_ERR_INVALID and "N_kv" in msg
+
+
+def test_entry_takes_one_row_per_query():
+    rc, msg = _entry(1, 64, 16, 64, 67, 16, 3, 16)  # (goes on to the workspace check)
+    assert rc == _lib.SI_ERR_INVALID and "workspace" in msg
