@@ -220,9 +220,10 @@ def csa_row_len(B: int, S: int, n_win: int, top_k: int, n_compressed: int, m: in
 
 
 def _row_len(B: int, S: int, n_win: int, cap: int, m: int, device) -> torch.Tensor:
-    """``[B, S]`` int32 ``n_win + min(cap, (s+1)//m)`` (one kernel; on other devices torch ops)."""
-    device = torch.device(device)
-    if device.type != "cuda" or n_win < 0 or cap < 0 or m <= 0:
+    """``[B, S]`` int32 ``n_win + min(cap, (s+1)//m)``: one kernel for the int32 sizes of a GPU, torch ops for the rest
+    (other devices or the default one, an ``m`` that is not an int, as ``S / T`` is not)."""
+    small = all(isinstance(v, int) and 0 <= v < 1 << 30 for v in (n_win, cap, m)) and m > 0
+    if device is None or torch.device(device).type != "cuda" or not small:
         s = torch.arange(S, device=device)
         return (n_win + torch.clamp((s + 1) // m, max=cap)).to(torch.int32).expand(B, S)
     out = torch.empty((S,), dtype=torch.int32, device=device)

@@ -272,3 +272,21 @@ def test_row_lengths(cuda_device, S, n_win, cap, m):
                 hca_row_len(2, S, n_win, cap, m, "cuda")):
         assert got.dtype == torch.int32 and torch.equal(got.cpu(), want)
     assert torch.equal(csa_row_len(2, S, n_win, cap, cap, m, "cpu"), want)
+
+
+@pytest.mark.parametrize("m", [4.0, 2.5, 1 << 40])
+def test_row_lengths_of_other_ratios(cuda_device, m):
+    # (S / T is a float; a ratio past int32 leaves the window only)
+    from streamindex_amd.csa import csa_row_len
+    from streamindex_amd.hca import hca_row_len
+
+    S, n_win, cap = 300, 16, 50
+    want = (n_win + torch.clamp((torch.arange(S) + 1) // m, max=cap)).to(torch.int32).expand(2, S)
+    for got in (csa_row_len(2, S, n_win, cap, cap, m, "cuda"), hca_row_len(2, S, n_win, cap, m, "cuda")):
+        assert got.is_cuda and got.dtype == torch.int32 and torch.equal(got.cpu(), want)
+
+
+def test_flash_csa_forward_takes_a_float_ratio(cuda_device):
+    q, kv, kvc, qi, ki, w, sink = _csa_inputs(1, 64, 16, 64, 16, 32, 4, seed=405)
+    o = flash_csa_forward(q, kv, kvc, qi, ki, w, sink, n_win=16, top_k=8, m=64 / kvc.shape[1])
+    assert torch.equal(o, flash_csa_forward(q, kv, kvc, qi, ki, w, sink, n_win=16, top_k=8, m=4))

@@ -72,3 +72,12 @@ def test_entry_refuses_other_row_counts(N):
 def test_entry_takes_one_row_per_query():
     rc, msg = _entry(1, 64, 16, 64, 67, 16, 3, 16)  # (goes on to the workspace check)
     assert rc == _lib.SI_ERR_INVALID and "workspace" in msg
+
+
+def test_row_lengths_on_the_default_device():
+    from streamindex_amd.csa import csa_row_len
+
+    want = 4 + torch.clamp((torch.arange(10) + 1) // 2, max=3)
+    for got in (csa_row_len(2, 10, 4, 3, 5, 2, None), csa_row_len(2, 10, 4, 3, 5, 2, "cpu"),
+                hca.hca_row_len(2, 10, 4, 3, 2, None)):
+        assert got.dtype == torch.int32 and torch.equal(got, want.to(torch.int32).expand(2, 10))
