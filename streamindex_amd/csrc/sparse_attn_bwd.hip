@@ -1228,22 +1228,23 @@ extern "C" int si_hca_attn_bwd(const void* q, const int64_t* q_strides, const vo
     return set_error(SI_ERR_INVALID, "tensors and the workspace must be 16-byte aligned");
   if (((S + T - 1) * kv_strides[1] + D) / 8 >= (int64_t{1} << 32))
     return set_error(SI_ERR_UNSUPPORTED, "kv batch larger than 64 GiB");
-  // (head offsets inside a row are 32-bit)
-  if (q_strides[2] < 0 || do_strides[2] < 0 || q_strides[2] >= (int64_t{1} << 24) || do_strides[2] >= (int64_t{1} << 24))
+  // (head offsets inside a row are 32-bit; a single head has none, whatever its stride)
+  const int64_t qsh = H > 1 ? q_strides[2] : 0, gsh = H > 1 ? do_strides[2] : 0;
+  if (qsh < 0 || gsh < 0 || qsh >= (int64_t{1} << 24) || gsh >= (int64_t{1} << 24))
     return set_error(SI_ERR_UNSUPPORTED, "head stride outside the aligned path");
   HcaPlan pl{};
   if (workspace_bytes < 0 || !hca_plan(B, S, H, D, n_win, T, static_cast<size_t>(workspace_bytes), &pl))
     return set_error(SI_ERR_INVALID, "workspace too small (see si_hca_attn_bwd_workspace_bytes)");
   AttnBwdArgs a{};
   a.q = static_cast<const uint16_t*>(q);
-  a.qsb = q_strides[0]; a.qss = q_strides[1]; a.qsh = q_strides[2];
+  a.qsb = q_strides[0]; a.qss = q_strides[1]; a.qsh = qsh;
   a.kv = static_cast<const uint16_t*>(kv);
   a.kvsb = kv_strides[0]; a.kvsn = kv_strides[1];
   a.sink = attn_sink;
   a.o = static_cast<const uint16_t*>(o);
   a.osb = o_strides[0]; a.oss = o_strides[1]; a.osh = o_strides[2];
   a.dout = static_cast<const uint16_t*>(dout);
-  a.gsb = do_strides[0]; a.gss = do_strides[1]; a.gsh = do_strides[2];
+  a.gsb = do_strides[0]; a.gss = do_strides[1]; a.gsh = gsh;
   a.lse = lse;
   a.lsb = lse_strides[0]; a.lss = lse_strides[1]; a.lsh = lse_strides[2];
   a.dq = static_cast<uint16_t*>(dq);

@@ -111,7 +111,8 @@ def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_w
         if ws is None:
             topk_idxs, row_len = _rows(B, S, n_win, n_compressed, m_prime, q.device)
             return sparse_attn_bwd(q, kv, attn_sink, topk_idxs, o, lse, do, softmax_scale, row_len=row_len)
-        q, o, do = (t if _aligned(t) and 0 <= t.stride(2) < 1 << 24 else t.contiguous() for t in (q, o, do))
+        # (the stride of a single head is not used, and contiguous() would leave it as it is)
+        q, o, do = (t if _aligned(t) and (H == 1 or 0 <= t.stride(2) < 1 << 24) else t.contiguous() for t in (q, o, do))
         attn_sink = attn_sink.contiguous()
         dq, dkv = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty_like(kv)
         dsink = torch.empty((H,), dtype=torch.float32, device=q.device)

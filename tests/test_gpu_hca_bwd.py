@@ -130,3 +130,15 @@ def test_kv_of_another_length(cuda_device, n1):
     o, lse = sparse_attn_fwd(q, full, sink, rows, row_len=row_len)
     dq, dkv, ds = sparse_attn_bwd(q, full, sink, rows, o, lse, do, row_len=row_len)
     _check(got, (dq, dkv[:, :n1], dkv[:, n1:], ds), 0.0, f"{n1} kv rows")
+
+
+def test_single_head_with_a_long_stride(cuda_device):
+    # one head of a [B, H, S, D] tensor seen as [B, S, H, D]: at S x D >= 2^24 its head stride passes the
+    # kernels' 32-bit head offsets, which a single head does not use
+    B, S, H, D, T, n_win, m = 1, 70, 1, 64, 4, 24, 16
+    q, kv, kvc, sink, do = _inputs(B, S, H, D, T, torch.bfloat16, 3)
+    long = q.as_strided(q.shape, (S * D, D, 1 << 25, 1))
+    leaves = [t.detach().requires_grad_(True) for t in (long, kv, kvc, sink)]
+    o = flash_hca_forward(*leaves, n_win=n_win, m_prime=m)
+    got = torch.autograd.grad(o, leaves, do.as_strided(do.shape, long.stride()))
+    assert all(torch.equal(x, y) for x, y in zip(got, _grads(q, kv, kvc, sink, do, n_win, m)))

@@ -81,3 +81,10 @@ def test_row_lengths_on_the_default_device():
     for got in (csa_row_len(2, 10, 4, 3, 5, 2, None), csa_row_len(2, 10, 4, 3, 5, 2, "cpu"),
                 hca.hca_row_len(2, 10, 4, 3, 2, None)):
         assert got.dtype == torch.int32 and torch.equal(got, want.to(torch.int32).expand(2, 10))
+
+
+def test_entry_ignores_the_stride_of_a_single_head():
+    rc, msg = _entry(1, 64, 1, 64, 67, 16, 3, 16, hs=1 << 25)
+    assert rc == _lib.SI_ERR_INVALID and "workspace" in msg
+    rc, msg = _entry(1, 64, 2, 64, 67, 16, 3, 16, hs=1 << 25)
+    assert rc == _lib.SI_ERR_UNSUPPORTED and "head stride" in msg
