@@ -7,11 +7,14 @@
 // MFMA accumulators, so nothing is written per pair:
 //   1. hca_bwd_idx_kernel: index rows whose window part starts at a multiple of
 //      32 keys, so that slot tile i of query s holds the aligned key tile
-//      (s-n_win+1)/32 + i whatever s is.
+//      (s-n_win+1)/32 + i whatever s is.  A masked slot names a key that the
+//      query attends to (as ~key): its row is gathered in the slot's place, so
+//      that 0 times a value that is not finite comes only from the query's own keys.
 //   2. sparse_attn_bwd_rows_kernel on those rows: dq, dsink terms, and P / dS of
 //      every tile (8 KiB each) in its register layout.
 //   3. hca_bwd_dkv_kernel: per (128 keys, RB query rows) the sum over the rows'
-//      heads of dS q + P dO, fp32, to a partial buffer.
+//      heads of dS q + P dO, fp32, to a partial buffer.  Sums that are not finite
+//      are taken again row by row, with only the keys each row attends to.
 //   4. hca_bwd_reduce_kernel: each key's partials in block order.
 // Every sum has a fixed order, so repeated calls are bit-identical.
 //
@@ -65,7 +68,9 @@ __device__ __forceinline__ void hca_item_rows(const HcaBwdArgs& h, int blk, int 
 
 // Index rows [S, 32 wtiles + T] and their used lengths [S], shared by all
 // batches: window column j of query s holds key 32 floor((s-n_win+1)/32) + j
-// where that lies in the window, then compressed entry i as S + i, else -1.
+// where that lies in the window, then legal compressed entry i as S + i, else ~key
+// of a key that the query attends to: s, or without a window the first entry
+// (a row without either has length 0).
 __global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t* row_len, int S, int n_win, int T, int m,
                                                           int wtiles) {
   const int s = blockIdx.x;
@@ -73,14 +78,15 @@ __global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t*
   const int first = s - n_win + 1;
   const int base = (first >> 5) * 32;
   const int legal = (s + 1) / m < T ? (s + 1) / m : T;
+  const int masked = ~(n_win > 0 ? s : S);
   for (int j = threadIdx.x; j < K; j += 256) {
     int v;
     if (j < 32 * wtiles) {
       const int t = base + j;
-      v = t >= 0 && t >= first && t <= s ? t : -1;
+      v = t >= 0 && t >= first && t <= s ? t : masked;
     } else {
       const int i = j - 32 * wtiles;
-      v = i < legal ? S + i : -1;
+      v = i < legal ? S + i : masked;
     }
     idx[static_cast<int64_t>(s) * K + j] = v;
   }
@@ -125,12 +131,14 @@ __device__ __forceinline__ void hca_copy16(const uint16_t* src, char* dst) {
 // the copies, the fragment reads behind the barrier and the MFMAs follow one
 // another.  Two more stages in flight (a ring of four) measured 1.39, touching
 // the lines two rows ahead or spreading the copies over the blocks nothing.
+// (waves per SIMD: two workgroups fit a CU up to D = 256, one above)
 template <int D, bool F16>
-__global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdArgs h) {
+__global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdArgs h) {
   using HS = HcaDkvShape<D>;
   constexpr int MBW = HS::MBW;
   __shared__ __attribute__((aligned(16))) char qd_lds[2 * HS::BUF];
   __shared__ __attribute__((aligned(16))) char coef_lds[HS::COEF];
+  __shared__ int nonfinite_lds[HS::NW];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -283,19 +291,104 @@ __global__ __launch_bounds__(512) void hca_bwd_dkv_kernel(AttnBwdArgs a, HcaBwdA
       }
       attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
     }
+    float z = 0.f;  // NaN where a sum is not finite
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
 #pragma unroll
       for (int nb = 0; nb < 8; nb += 2) mfma_result_fence(acc[m][nb], acc[m][nb + 1]);
+      if (blk_lo + m < HS::MBT) {  // (at D = 32 waves 2 and 3 hold no block of the row)
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) z = __builtin_fmaf(acc[m][nb][c], 0.f, z);
+      }
     }
     // lane (key 16 nb + i16 of the group, g) holds dimensions 16 mbi + 4 g + 0..3
     float* out = h.part + static_cast<int64_t>(item) * kHcaKeys * D;
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
-      if (blk_lo + m < HS::MBT) {  // (at D = 32 waves 2 and 3 hold no block of the row)
+      if (blk_lo + m < HS::MBT) {
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb)
           *reinterpret_cast<f32x4*>(out + (nb * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = acc[m][nb];
+      }
+    }
+    const bool bad = __builtin_amdgcn_ballot_w64(z != 0.f) != 0;
+    if (lane == 0) nonfinite_lds[wave] = bad ? 1 : 0;
+    attn_tile_barrier();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < HS::NW; ++w) any |= nonfinite_lds[w];
+    if (__builtin_amdgcn_readfirstlane(any) != 0) {
+      // The coefficients of the keys that a row does not attend to are 0, and 0
+      // times an infinity or NaN of the row's Q or dO is NaN.  So: one dimension
+      // block and KH of the group's 16-key blocks at a time (no more registers than
+      // the loop above takes), a row's sum over its heads apart, added for the keys
+      // that the row attends to.  (8 / KH MBW passes over the stages instead of one.)
+      constexpr int KH = 4;
+      for (int pass = 0; pass < 8 / KH * MBW; ++pass) {
+        const int m = pass / (8 / KH), n0 = pass % (8 / KH) * KH;
+        const bool has = m < NB;
+        const uint32_t ca = cf0 + n0 * HS::CW4;
+        f32x4 row[KH], tot[KH];
+#pragma unroll
+        for (int nb = 0; nb < KH; ++nb) row[nb] = tot[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        cur = Stage{r0, 0};
+        copy_stage(cur, 0);
+        load_coef(cur);
+        for (buf = 0; cur.s < r1; buf ^= 1) {
+          __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));
+          *reinterpret_cast<u32x4*>(cst) = cf;
+          attn_tile_barrier();
+          const Stage at = cur;
+          cur = next(cur);
+          if (cur.s < r1) {
+            copy_stage(cur, buf ^ 1);
+            load_coef(cur);
+          }
+          if (has) {
+            v4i16 blo[KH], bhi[KH];
+            attn_static_for<0, KH>([&](auto NC) {
+              constexpr int nb = decltype(NC)::value;
+              constexpr int off = (nb >> 1) * 2 * HS::CW4 + 8 * (nb & 1);
+              blo[nb] = tr_read<off>(ca);
+              bhi[nb] = tr_read<off + 64>(ca);
+            });
+            const uint32_t qa = qd0 + buf * HS::BUF + m * 32;
+            v4i16 alo = tr_read<0>(qa);
+            v4i16 ahi = tr_read<4 * HS::QROW>(qa);
+            lds_wait_n<0>();
+            reg_tie(alo);
+            reg_tie(ahi);
+            const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo, ahi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int nb = 0; nb < KH; ++nb) {
+              reg_tie(blo[nb]);
+              reg_tie(bhi[nb]);
+              const bf16x8 bf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[nb], bhi[nb], 0, 1, 2, 3, 4, 5, 6, 7));
+              if (at.part == 0) row[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+              row[nb] = mfma16x16x32<F16>(af, bf, row[nb]);
+            }
+            if (at.part == nq - 1) {
+#pragma unroll
+              for (int nb = 0; nb < KH; nb += 2) mfma_result_fence(row[nb], row[nb + 1]);
+#pragma unroll
+              for (int nb = 0; nb < KH; ++nb) {
+                const int key = kt * 32 + (n0 + nb) * 16 + i16;
+                const bool attends = window ? key <= at.s && key > at.s - h.n_win
+                                            : key < h.T && static_cast<int64_t>(h.m) * (key + 1) <= at.s + 1;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tot[nb][c] = attends ? tot[nb][c] + row[nb][c] : tot[nb][c];
+              }
+            }
+          }
+          attn_tile_barrier();
+        }
+        if (has && blk_lo + m < HS::MBT) {
+#pragma unroll
+          for (int nb = 0; nb < KH; ++nb)
+            *reinterpret_cast<f32x4*>(out + ((n0 + nb) * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = tot[nb];
+        }
       }
     }
   };
@@ -428,6 +521,7 @@ static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs
   a.rlss = 1;
   a.K = K;
   a.ntiles = pl.ntiles;
+  a.masked_keys = 1;
   a.dsink_rows = reinterpret_cast<float*>(ws + pl.dsink_rows);
   a.coef = reinterpret_cast<uint16_t*>(ws + pl.coef);
   h.wtiles = pl.wtiles;

@@ -73,6 +73,7 @@ struct AttnBwdArgs {
   int nrows;           // rows in this chunk
   float scale, scale_log2;
   int f16;             // element type: 0 bf16, 1 fp16
+  int masked_keys;     // a masked slot's index is ~key of the row to gather in its place (0: key 0's)
 };
 
 constexpr int kBwdThreads = 2 * kAttnWaves * 64;
@@ -292,7 +293,9 @@ __global__ __launch_bounds__(kBwdThreads) void sparse_attn_bwd_rows_kernel(AttnB
         const int j = t * kAttnTK + lane;
         const bool ok = j < klen && raw >= 0 && raw < a.N;
         bias_lds[slot][lane] = ok ? 0.f : -__builtin_inff();
-        rowoff_lds[slot][lane] = static_cast<uint32_t>((ok ? raw : 0) * (a.kvsn / 8));
+        // (a slot past the row re-reads the row's last index, valid or not)
+        const int64_t masked = a.masked_keys ? (raw < 0 ? ~raw : raw) : 0;
+        rowoff_lds[slot][lane] = static_cast<uint32_t>((ok ? raw : masked) * (a.kvsn / 8));
       }
     };
     // Gather of tile t: LDS slot e (16 bytes) holds chunk (e % CPR) ^ f(key)

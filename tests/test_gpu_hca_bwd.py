@@ -142,3 +142,42 @@ def test_single_head_with_a_long_stride(cuda_device):
     o = flash_hca_forward(*leaves, n_win=n_win, m_prime=m)
     got = torch.autograd.grad(o, leaves, do.as_strided(do.shape, long.stride()))
     assert all(torch.equal(x, y) for x, y in zip(got, _grads(q, kv, kvc, sink, do, n_win, m)))
+
+
+def _same_spread(got, ref, eps, label):
+    """Not finite in the same places, equal elsewhere."""
+    for x, y, name in zip(got, ref, ("dq", "dkv", "dkv_compressed", "dsink")):
+        fin = torch.isfinite(y)
+        assert torch.equal(torch.isfinite(x), fin), f"{label} {name}: not finite elsewhere"
+        _check((torch.where(fin, x, 0),), (torch.where(fin, y, 0),), eps, f"{label} {name}")
+
+
+@pytest.mark.parametrize("D,n_win,T,m,H", [(64, 40, 20, 8, 20), (576, 128, 2, 128, 64), (32, 0, 60, 4, 16),
+                                           (256, 33, 0, 1, 130)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_non_finite_rows_stay_with_their_keys(cuda_device, D, n_win, T, m, H, value):
+    # one element of one query's q, and of another's do: only the keys that these queries attend to take it up
+    B, S = 2, 300
+    q, kv, kvc, sink, do = _inputs(B, S, H, D, T, torch.bfloat16, D)
+    q[0, 100, H - 1, 3] = value
+    do[1, 250, 0, D - 1] = value
+    x = (q, kv, kvc, sink, do)
+    ref = _general(*x, n_win, m)
+    assert all((~torch.isfinite(r)).any() and torch.isfinite(r).any() for r in ref[:1 + (n_win > 0)])
+    _same_spread(_grads(*x, n_win, m), ref, 2 ** -8, f"D={D},n_win={n_win},T={T}")
+
+
+@pytest.mark.parametrize("n_win,T,m", [(64, 0, 4), (32, 32, 1), (0, 32, 2)])
+def test_non_finite_keys_stay_with_their_rows(cuda_device, n_win, T, m):
+    # a masked slot gathers some row in its place, whose infinities times a weight of 0 must not reach dq
+    B, S, H, D = 1, 300, 16, 64
+    x = _inputs(B, S, H, D, T, torch.bfloat16, n_win)
+    x[1][0, 0] = float("inf")
+    if T:
+        x[2][0, 7] = float("nan")
+    got, ref = _grads(*x, n_win, m), _general(*x, n_win, m)
+    for s in range(S):
+        if torch.isfinite(ref[0][0, s]).all():
+            assert torch.isfinite(got[0][0, s]).all(), f"dq of query {s}"
+    keys = [torch.isfinite(r).all(dim=2)[0] for r in ref[1:3]]
+    assert all((torch.isfinite(g).all(dim=2)[0] | ~k).all() for g, k in zip(got[1:3], keys))
