@@ -537,10 +537,15 @@ void indexer_topk_kernel(IndexerArgs a) {
 
 // ---------------------------------------------------------------------------
 // Materialised score matrix [B, S, T] fp32 (no mask, as the reference kernel).
-// The grid's y axis splits the keys into chunks of score_tiles tiles.
+// The grid's y axis splits the keys into chunks of score_tiles tiles: a
+// workgroup's keys, scores and T start at its chunk, so that the loop is that of
+// a whole row (with a first tile in its counters it took 135 registers instead of
+// 117 at H <= 32, D = 64, and one workgroup a CU instead of two: T = 8,000,
+// S = 4 x 1,500, H = 16 239 us instead of 198).
 // ---------------------------------------------------------------------------
 template <int HB, int D, int NW, int TILE_N>
-__global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a) {
+__global__ __launch_bounds__(NW * 64, D == 32 && HB == 2 ? 4 : 1)  // (4: two workgroups a CU, two registers fewer than it would take)
+void indexer_score_kernel(IndexerArgs a) {
   constexpr int NT = NW * 64;
   constexpr int NB = TILE_N / 32;
   constexpr int TILE_BYTES = TILE_N * D * 2;
@@ -556,21 +561,21 @@ __global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a
   QueryFrags<HB, D> qfr;
   if (active) qfr.load(a, b, s, lane);
 
-  const uint16_t* kb = a.k + b * a.ksb;
-  float* orow = a.scores + b * a.ssb + static_cast<int64_t>(active ? s : 0) * a.sss;
+  const int t0 = static_cast<int>(blockIdx.y) * a.score_tiles * TILE_N;
+  const int T = a.T - t0 < a.score_tiles * TILE_N ? a.T - t0 : a.score_tiles * TILE_N;
+  const uint16_t* kb = a.k + b * a.ksb + static_cast<int64_t>(t0) * a.kst;
+  float* orow = a.scores + b * a.ssb + static_cast<int64_t>(active ? s : 0) * a.sss + static_cast<int64_t>(t0) * a.sst;
 
   KTileLoader<D, TILE_N, NT> ld;
   ld.init(a.kst);
-  const int it0 = static_cast<int>(blockIdx.y) * a.score_tiles;
-  const int left = (a.T + TILE_N - 1) / TILE_N - it0;
-  const int ntiles = it0 + (left < a.score_tiles ? left : a.score_tiles);
-  if (it0 < ntiles) ld.issue(kb, a.kst, it0 * TILE_N, a.T, lds);
+  const int ntiles = (T + TILE_N - 1) / TILE_N;
+  if (ntiles > 0) ld.issue(kb, a.kst, 0, T, lds);
   tile_barrier();
   static_assert(NB % 2 == 0, "32-key blocks are stored in pairs");
-  for (int it = it0; it < ntiles; ++it) {
+  for (int it = 0; it < ntiles; ++it) {
     const bool more = it + 1 < ntiles;
-    if (more) ld.issue(kb, a.kst, (it + 1) * TILE_N, a.T, lds + ((it + 1 - it0) & 1) * TILE_BYTES);
-    const char* tile = lds + ((it - it0) & 1) * TILE_BYTES;
+    if (more) ld.issue(kb, a.kst, (it + 1) * TILE_N, T, lds + ((it + 1) & 1) * TILE_BYTES);
+    const char* tile = lds + (it & 1) * TILE_BYTES;
     const int tbase = it * TILE_N;
     // Full tiles of a row that overwrites its scores issue exactly NB / 2
     // stores after the copy of tile it+1, so the wait before the barrier
@@ -578,9 +583,9 @@ __global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a
     // operations -- global loads, LDS-DMA copies, stores -- report completion
     // to the wave in execution order on this GFX9-family part, which is what
     // vmcnt counts); every other case waits for all.
-    const bool lean = active && !a.accumulate && tbase + TILE_N <= a.T;
+    const bool lean = active && !a.accumulate && tbase + TILE_N <= T;
     if (active) {
-      int nblk = (a.T - tbase + 31) / 32;
+      int nblk = (T - tbase + 31) / 32;
       nblk = nblk > NB ? NB : nblk;
       float p[NB];
       if (nblk == NB) {
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(NW * 64, 1) void indexer_score_kernel(IndexerArgs a
         float* o = orow + static_cast<int64_t>(t) * a.sst;
         if (lean) {
           *o = v;
-        } else if (t < a.T) {
+        } else if (t < T) {
           *o = a.accumulate ? *o + v : v;
         }
       }
