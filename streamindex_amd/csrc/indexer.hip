@@ -8,11 +8,10 @@ namespace si {
 
 int g_topk_kernel_mode = 0;
 
-// When the few-row top-k runs (few_plan): at most kFewMaxGroups four-row
-// groups (one per CU), rows of at least kFewMinKeys keys, no causal ratio (its
-// rows are short while they are few), and a scratch within kFewMaxScratch.
-// us a call, one-wave-per-row kernel against this one, H = 64, D = 128,
-// k = 512 (22 us is the host's share of a call):
+// When the few-row top-k runs (few_worth): at most kFewMaxGroups four-row groups
+// (one per CU), no causal ratio (its rows are short while they are few), and a
+// scratch within kFewMaxScratch.  us a call (17 to 20 of them are the host's),
+// one-wave-per-row kernel against this one, H = 64, D = 128, k = 512:
 //   rows x keys   1 x 1,024   30 -> 22     4 x 16,384 (four batches)  203 -> 23
 //   1 x 65,536   754 -> 27    1 x 262,144  2,910 -> 35
 //   256 x 8,192  146 -> 45    512 x 32,768  460 -> 263
@@ -20,7 +19,6 @@ int g_topk_kernel_mode = 0;
 // and past the line 1,536 x 2,048  79 -> 85, 2,048 x 32,000  818 -> 916: there
 // the one-wave-per-row kernel fills the chip and saves the scores' round trip.
 constexpr int64_t kFewMaxGroups = 256;
-constexpr int kFewMinKeys = 1024;
 constexpr int64_t kFewMaxScratch = int64_t(256) << 20;
 
 // Kernel and selection capacity for a top-k shape.  A compaction keeps
@@ -149,11 +147,33 @@ struct FewPlan {
   int64_t bytes;    // scratch: scores, then the segments' keys
 };
 
+// Whether the two passes are the faster ones (see kFewMaxGroups).  The lines, us of
+// the one-wave-per-row kernel against the two passes on both sides:
+//   * below 8 rows a batch each row reads the keys for itself, so its count of rows
+//     is limited, not its groups: 256 x 1 row x 30,000 keys 426, 426 (D = 256: 691,
+//     919; 128 x 1: 658, 497), 64 x 7 x 30,000 436, 510, 256 x 4 x 12,000 248, 501;
+//   * a row costs more of the chip at D = 256 and from three head blocks on, which
+//     the one-wave kernel fills with fewer rows: 1,024 x 30,000, D = 256 816, 911
+//     (512 rows 691, 484); 128 x 8 x 12,000, H = 128 346, 401 (4,096 keys 137, 141);
+//   * short rows of few picks, which the one-wave kernel hardly compacts: k = 16,
+//     one row x 1,024 keys, H = 8 17, 20 (2,048 keys 24, 21); 1,024 rows x 3,000, H = 64
+//     55, 64 (x 4,096, H = 8 55, 45); k = 128, one x 1,024, H = 32 18, 20 (2,048 27, 21).
+static bool few_worth(const IndexerArgs& a, int D) {
+  const int64_t rows = static_cast<int64_t>(a.B) * a.S;
+  const int64_t groups = static_cast<int64_t>(a.B) * ((a.S + 3) / 4);
+  const bool many = groups > kFewMaxGroups / 2;
+  const int HB = (a.H + 31) / 32;
+  if (groups > kFewMaxGroups) return false;
+  if (a.S < 8 && rows > (D == 256 ? kFewMaxGroups / 2 : kFewMaxGroups)) return false;
+  if (many && (D == 256 || (a.S >= 8 && HB >= 3 && a.T >= 8192))) return false;
+  if (a.top_k >= 256 || HB >= 3) return a.T >= 1024;
+  return a.T >= (many && a.top_k <= 64 ? 4096 : 2048);
+}
+
 static FewPlan few_plan(const IndexerArgs& a, int D) {
   FewPlan f{};
   TopkPlan p{};
-  if (g_topk_kernel_mode != 0 || a.ratio > 0 || a.T < kFewMinKeys) return f;
-  if (static_cast<int64_t>(a.B) * ((a.S + 3) / 4) > kFewMaxGroups) return f;
+  if (g_topk_kernel_mode != 0 || a.ratio > 0 || !few_worth(a, D)) return f;
   if (plan_topk(a, D, &p) != SI_OK || p.kernel == TOPK_SPLIT) return f;
   const int64_t rows = static_cast<int64_t>(a.B) * a.S;
   f.sstride = (static_cast<int64_t>(a.T) + 63) / 64 * 64;

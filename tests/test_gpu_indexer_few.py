@@ -1,8 +1,8 @@
 """The two-pass top-k for few query rows over many keys (indexer_topk_few.h).
 
-Calls with at most 256 four-row groups and 1,024 or more keys, without a
-causal ratio, write their scores to a scratch and select with one workgroup
-per row (and segment of 16,384 keys).  Scores are formed by the same fp32
+Calls with at most 256 four-row groups and 1,024 or more keys (few_worth draws
+the line more closely), without a causal ratio, write their scores to a scratch
+and select with one workgroup per row (and segment of 16,384 keys).  Scores are formed by the same fp32
 operations and ranked by the same keys as in the one-wave-per-row kernel, so
 every case compares the two for exact equality; two also go through the
 oracle gate of tests/indexer_check.py.  Cases: both score kernels (below and
@@ -108,3 +108,42 @@ def test_plan_lines(cuda_device):
     assert not _uses_scratch(1, 1, 4096, 64, 128, 2049)      # head-split shapes
     assert not _uses_scratch(1, 1, 4096, 192, 128, 512)
     assert _lib.load().si_indexer_topk_scratch_bytes(1, 512, 4096, 64, 128, 512, 4) == 0
+
+
+@pytest.mark.parametrize("B,S,T,H,D,k,few", [
+    (256, 1, 30000, 64, 128, 512, True),     # rows, not groups, below 8 rows a batch
+    (64, 7, 30000, 64, 128, 512, False),
+    (256, 4, 4096, 32, 128, 512, False),
+    (128, 1, 30000, 64, 256, 512, True),     # D = 256 and three or four head blocks fill the chip earlier
+    (129, 1, 30000, 64, 256, 512, False),
+    (1, 512, 30000, 64, 256, 512, True),
+    (1, 516, 30000, 64, 256, 512, False),
+    (1, 1024, 4096, 128, 128, 512, True),
+    (1, 1024, 8192, 128, 128, 512, False),
+    (1, 1, 1024, 32, 128, 128, False),       # short rows of few picks
+    (1, 1, 2048, 32, 128, 128, True),
+    (1, 1024, 2048, 64, 128, 16, False),
+    (1, 1024, 4096, 64, 128, 16, True),
+])
+def test_plan_lines_of_rows_heads_and_picks(cuda_device, B, S, T, H, D, k, few):
+    assert _uses_scratch(B, S, T, H, D, k) == few
+
+
+@pytest.mark.parametrize("T,k", [(4096, 300), (16384, 512), (40000, 512)])
+def test_scores_that_are_not_finite(narrow, T, k):
+    # infinities and NaN among the scores, in rows of every kind of them: the order of their bits, as in the other kernel
+    S, H, D = 6, 32, 64
+    q, ki, w = synth.indexer_inputs(1, S, H, D, T, seed=T)
+    g = torch.Generator().manual_seed(T)
+    at = torch.randperm(T, generator=g)[:900]
+    ki[0, at[:300].cuda(), 0] = float("inf")
+    ki[0, at[300:600].cuda(), 1] = float("-inf")
+    q[0, 1, :, :2] = 0.5                   # +inf and -inf scores
+    q[0, 2, :, :2] = 0                     # 0 times infinity
+    w[0, 3] = -w[0, 3].abs()               # -inf
+    w[0, 4, 0] = float("nan")              # a row of NaN
+    w[0, 5] = 0                            # zeros and NaN
+    a, b = chunked_indexer_topk(q, ki, w, k), narrow(lambda: chunked_indexer_topk(q, ki, w, k))
+    assert torch.equal(a[0], b[0])
+    assert torch.equal(a[1].view(torch.int32), b[1].view(torch.int32))
+    assert not torch.isfinite(a[1]).all()
