@@ -338,12 +338,10 @@ struct PoolArgs {
 // Bound: HBM.  Every score and content row is read once, 16 bytes a lane
 // (N = 8, fp32: 4), U scores and U contents in flight per thread, with the
 // running maximum moved once a chunk (an entry of up to U rows never rescales).
-// R = 8 where entries are long and few (m = 128), so that enough loads are in
-// flight.  N = 1 serves the channel counts and addresses that are not whole
-// 16-byte vectors.
-template <int DT, int N, int R>
+// N = 1 serves the channel counts and addresses that are not whole 16-byte
+// vectors.  R and U: launch_compress.
+template <int DT, int N, int R, int U>
 __global__ __launch_bounds__(256) void token_compress_kernel(PoolArgs p) {
-  constexpr int U = 8;
   constexpr int ITEMS = 256 / R;
   const int local = static_cast<int>(threadIdx.x) % ITEMS;
   const int part = static_cast<int>(threadIdx.x) / ITEMS;
@@ -490,14 +488,38 @@ template <int DT> struct Fp4Sim { static constexpr auto fn = fp4_simulate_kernel
 template <int DT> struct Fp8Pack { static constexpr auto fn = fp8_pack_kernel<DT>; };
 template <int DT> struct Fp4Pack { static constexpr auto fn = fp4_pack_kernel<DT>; };
 
-template <int DT, int N, int R>
+template <int DT, int N, int R, int U>
 static int launch_compress_r(const PoolArgs& p, hipStream_t st) {
   const int64_t items = p.B * p.nblk * (p.C / N);
   const int64_t blocks = (items + 256 / R - 1) / (256 / R);
   if (blocks > 0x7fffffffLL) return set_error(SI_ERR_UNSUPPORTED, "tensor too large");
   if (blocks == 0) return SI_OK;
-  hipLaunchKernelGGL((token_compress_kernel<DT, N, R>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((token_compress_kernel<DT, N, R, U>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, p);
   return check_launch("token_compress_kernel");
+}
+// Threads per item (R) and rows per chunk (U).  Loads in flight hide the memory
+// latency: an entry of more than U rows is split over several threads where the
+// items alone do not fill the GPU, and not where they do (each added thread costs a
+// share of an LDS exchange).  us, one thread against R (bf16, 16-byte vectors):
+//   S = 512, C = 64:  m = 2 x 24  19 -> 6 (R = 8), m = 12  6.8 -> 5.8 (2)
+//   S = 64K, C = 576:  m = 24  34 (1), 41 with R = 4;  m = 64  83 (before) -> 37 (8)
+//   S = 64K, C = 64:  m = 16  11 -> 6 (4)
+// Many single channels (N = 1) of few rows need no chunk at all, each chunk's unused
+// rows cost more than the rescales: S = 64K, C = 100, m = 1  33 -> 24, m = 16  16 -> 13.
+template <int DT, int N>
+static int launch_compress_n(const PoolArgs& p, hipStream_t st) {
+  const int64_t items = p.B * p.nblk * (p.C / N);
+  const int64_t rows = p.overlap ? 2 * p.m : p.m;
+  if (N == 1 && rows <= 32 && items >= (3 << 16)) return launch_compress_r<DT, N, 1, 1>(p, st);
+  int R = 1;
+  if (N > 1 && p.m >= 32) R = 8;
+  while (R < 8 && R * 8 < rows && items * R < (N == 1 ? 1 << 19 : 1 << 17)) R *= 2;
+  switch (R) {
+    case 1: return launch_compress_r<DT, N, 1, 8>(p, st);
+    case 2: return launch_compress_r<DT, N, 2, 8>(p, st);
+    case 4: return launch_compress_r<DT, N, 4, 8>(p, st);
+    default: return launch_compress_r<DT, N, 8, 8>(p, st);
+  }
 }
 template <int DT>
 static int launch_compress(const PoolArgs& p, hipStream_t st) {
@@ -506,9 +528,7 @@ static int launch_compress(const PoolArgs& p, hipStream_t st) {
                          reinterpret_cast<uintptr_t>(p.cb) | reinterpret_cast<uintptr_t>(p.zb) |
                          reinterpret_cast<uintptr_t>(p.ba) | reinterpret_cast<uintptr_t>(p.bb) |
                          reinterpret_cast<uintptr_t>(p.out);
-  if (p.C % N || (ptrs & 15)) return launch_compress_r<DT, 1, 1>(p, st);
-  // Long entries: several threads each, so that their rows load in parallel.
-  return p.m >= 32 ? launch_compress_r<DT, N, 8>(p, st) : launch_compress_r<DT, N, 1>(p, st);
+  return p.C % N || (ptrs & 15) ? launch_compress_n<DT, 1>(p, st) : launch_compress_n<DT, N>(p, st);
 }
 
 static int log2_lanes(int64_t bs) {

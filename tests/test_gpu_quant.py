@@ -91,7 +91,7 @@ def test_gated_pool(cuda_device):
     (True, 4, 44, 0),     # 44 channels are whole 16-byte vectors in fp32 only
     (True, 4, 37, 0),     # scalar kernel
     (True, 4, 96, 1),     # rows off the 16-byte grid: scalar kernel
-    (False, 31, 64, 0),   # longest entry of one thread
+    (False, 31, 64, 0),   # longest entry whose threads depend on the number of entries
     (False, 32, 64, 0),   # shortest entry of eight threads
     (False, 67, 72, 0),   # eight threads, uneven chunks, a partial workgroup
     (True, 33, 8, 0),
@@ -132,3 +132,32 @@ def test_fp4_pack_ties_signs_and_shift(cuda_device, dt):
         assert np.array_equal(O.fp4_unpack(p.cpu().numpy()), rv)
         b = p.cpu().numpy()
         assert not np.any((b & 0xF) == 8) and not np.any((b >> 4) == 8)  # zero has one code
+
+
+@pytest.mark.parametrize("dt,tol", [("float32", 1e-5), ("bfloat16", 2e-2)])
+@pytest.mark.parametrize("overlap,m,S,C,shift", [
+    (False, 7, 70, 64, 0),       # up to 8 rows: one thread an entry
+    (False, 9, 91, 64, 0),       # two threads
+    (True, 9, 91, 64, 0),        # four
+    (True, 31, 310, 64, 0),      # eight
+    (True, 9, 30000, 256, 0),    # enough entries to fill the GPU: one thread
+    (True, 31, 310, 37, 0),      # single channels: eight threads
+    (False, 1, 5400, 37, 0),     # and enough of them: row by row
+    (True, 16, 87000, 37, 0),
+    (False, 32, 3200, 64, 1),
+])
+def test_token_compressor_threads_per_entry(cuda_device, dt, tol, overlap, m, S, C, shift):
+    rng = np.random.default_rng(m + S)
+    arr = [O.round_to(rng.standard_normal((1, S, C)).astype(np.float32), dt) for _ in range(4 if overlap else 2)]
+    arr[1][:, m:2 * m] = -np.inf if m > 1 and overlap else arr[1][:, m:2 * m]
+    ba, bb = rng.standard_normal((m, C)).astype(np.float32), rng.standard_normal((m, C)).astype(np.float32)
+
+    def dev(a):
+        x = torch.from_numpy(a).to(TD[dt])
+        return torch.empty(x.numel() + shift, dtype=x.dtype, device="cuda")[shift:].view(x.shape).copy_(x)
+
+    t = [dev(a) for a in arr]
+    kw = dict(c_b=t[2], z_b=t[3], b_b=torch.from_numpy(bb).cuda()) if overlap else {}
+    got = compressor.token_compressor(t[0], t[1], torch.from_numpy(ba).cuda(), m, overlap=overlap, **kw)
+    ref = O.token_compressor(arr[0], arr[1], ba, m, *((arr[2], arr[3], bb) if overlap else (None, None, None)), overlap)
+    assert np.abs(got.float().cpu().numpy() - ref).max() <= tol * np.abs(ref).max()
