@@ -34,11 +34,11 @@ struct HcaBwdArgs {
   int n_win, m, T;
   int wtiles;      // 32-key window tiles of an index row
   int RB;          // query rows of a block (a multiple of 32)
-  int b0, nb;      // batches of this chunk
+  int b0;          // first batch of this chunk
   int s0, s1;      // query rows of this chunk (s0 a multiple of RB)
   int GW, ncg;     // window / compressed key groups of a block
   float* part;     // [nb, blocks, GW + ncg, kHcaKeys, D]
-  float* acc;      // [B, N, D] fp32 sums of the earlier chunks
+  float* acc;      // [N, D] fp32 sums of the batch's earlier chunks
   uint16_t* dkv;   // [B, N, D]
   int64_t dsb, dsn;
   int first, last;  // first / last chunk of the batch
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256) void hca_bwd_reduce_kernel(HcaBwdArgs h, int S
   if (from >= to && !h.first && !h.last) return;
   if (d >= D) return;
   f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
-  float* acc = h.acc + (static_cast<int64_t>(b) * N + n) * D + d;
+  float* acc = h.acc + static_cast<int64_t>(n) * D + d;  // (a batch in several chunks is alone in them)
   if (!h.first) sum = *reinterpret_cast<const f32x4*>(acc);
   if (from < to) {
     const int q0 = static_cast<int>(from) / h.RB, q1 = static_cast<int>(to - 1) / h.RB;  // inclusive
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(256) void hca_bwd_reduce_kernel(HcaBwdArgs h, int S
 // ---- host side ----------------------------------------------------------------
 struct HcaPlan {
   int64_t rows;  // query rows of a chunk (a multiple of RB, or S)
-  int64_t nb;    // batches of a chunk (all of them, or 1 where a batch takes several chunks)
+  int64_t nb;    // batches of a chunk (1 where a batch takes several chunks)
   int RB, wtiles, ntiles, GW, ncg;
   size_t dsink_rows, acc, idx, row_len, coef, part, total;
 };
@@ -471,7 +471,7 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   };
   const int64_t blocks = (rows + RB - 1) / RB;
   p->dsink_rows = take(B * S * 64 * HG * 4);
-  p->acc = take(rows < S ? B * (S + T) * D * 4 : 0);
+  p->acc = take(rows < S ? (S + T) * D * 4 : 0);
   p->idx = take(S * (32 * p->wtiles + T) * 4);
   p->row_len = take(S * 4);
   p->coef = take(nb * rows * HG * p->ntiles * kCoefTile * 2);
@@ -479,8 +479,11 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   p->total = off;
 }
 
-// The fewest chunks whose plan fits `bytes`; false when none does.  Row blocks
-// of 128 (fewer partials), smaller where that leaves CUs idle.
+// The fewest chunks whose plan fits `bytes`; false when none does: all batches, else
+// equal groups of whole batches, else equal parts of one batch's rows (which add up
+// dkv in the workspace).  Equal, because a short last chunk costs what a whole one
+// does on the CUs that it leaves idle.  Row blocks of 64 (fewer partials), smaller
+// where that leaves CUs idle.
 static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, size_t bytes, HcaPlan* p) {
   for (int RB = 64; RB >= 32; RB /= 2) {
     hca_plan_for(B, S, H, D, n_win, T, RB, S, B, p);
@@ -488,18 +491,29 @@ static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, 
   }
   if (p->total <= bytes) return true;
   const int RB = p->RB;
-  int64_t lo = 0, hi = (S + RB - 1) / RB;  // chunks of `lo` row blocks fit
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) / 2;
-    hca_plan_for(B, S, H, D, n_win, T, RB, mid * RB, 1, p);
-    if (p->total <= bytes) lo = mid; else hi = mid;
-  }
-  if (lo == 0) {
-    hca_plan_for(B, S, H, D, n_win, T, RB, S, 1, p);  // one chunk per batch
+  // The greatest x below `end` with fits(x) (0: none), then ceil(end / chunks of x).
+  auto share = [&](int64_t end, auto fits) {
+    int64_t lo = 0, hi = end;
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) / 2;
+      if (fits(mid)) lo = mid; else hi = mid;
+    }
+    if (lo == 0) return int64_t{0};
+    const int64_t chunks = (end + lo - 1) / lo;
+    return (end + chunks - 1) / chunks;
+  };
+  auto batches = [&](int64_t nb) {
+    hca_plan_for(B, S, H, D, n_win, T, RB, S, nb, p);
     return p->total <= bytes;
-  }
-  hca_plan_for(B, S, H, D, n_win, T, RB, lo * RB, 1, p);
-  return true;
+  };
+  auto blocks = [&](int64_t n) {
+    hca_plan_for(B, S, H, D, n_win, T, RB, n * RB, 1, p);
+    return p->total <= bytes;
+  };
+  const int64_t nb = share(B, batches);
+  if (nb > 0) return batches(nb);
+  const int64_t n = share((S + RB - 1) / RB, blocks);
+  return n > 0 && blocks(n);
 }
 
 template <int D, bool F16>
@@ -530,8 +544,8 @@ static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs
   h.ncg = pl.ncg;
   h.part = reinterpret_cast<float*>(ws + pl.part);
   h.acc = reinterpret_cast<float*>(ws + pl.acc);
-  h.nb = static_cast<int>(pl.nb);
   for (int64_t b0 = 0; b0 < a.B; b0 += pl.nb) {
+    const int64_t nb = a.B - b0 < pl.nb ? a.B - b0 : pl.nb;
     for (int64_t s0 = 0; s0 < S; s0 += pl.rows) {
       h.b0 = static_cast<int>(b0);
       h.s0 = static_cast<int>(s0);
@@ -539,17 +553,17 @@ static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs
       h.first = s0 == 0;
       h.last = h.s1 == S;
       a.row0 = b0 * S + s0;
-      a.nrows = static_cast<int>(pl.nb * (h.s1 - h.s0));
+      a.nrows = static_cast<int>(nb * (h.s1 - h.s0));
       const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(a.nrows) * a.HG);
       hipLaunchKernelGGL((sparse_attn_bwd_rows_kernel<D, false, F16>), dim3(grid), dim3(kBwdThreads), 0, st, a);
       if ((rc = check_launch("sparse_attn_bwd_rows_kernel"))) return rc;
       const int64_t blocks = (h.s1 + h.RB - 1) / h.RB - h.s0 / h.RB;
-      const unsigned items = static_cast<unsigned>(pl.nb * blocks * (h.GW + h.ncg));
+      const unsigned items = static_cast<unsigned>(nb * blocks * (h.GW + h.ncg));
       if (items > 0) {
         hipLaunchKernelGGL((hca_bwd_dkv_kernel<D, F16>), dim3(items), dim3(HcaDkvShape<D>::NW * 64), 0, st, a, h);
         if ((rc = check_launch("hca_bwd_dkv_kernel"))) return rc;
       }
-      hipLaunchKernelGGL((hca_bwd_reduce_kernel<D, F16>), dim3(static_cast<unsigned>(pl.nb * (S + h.T))), dim3((D / 4 + 63) / 64 * 64), 0,
+      hipLaunchKernelGGL((hca_bwd_reduce_kernel<D, F16>), dim3(static_cast<unsigned>(nb * (S + h.T))), dim3((D / 4 + 63) / 64 * 64), 0,
                          st, h, S);
       if ((rc = check_launch("hca_bwd_reduce_kernel"))) return rc;
     }

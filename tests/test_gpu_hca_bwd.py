@@ -181,3 +181,31 @@ def test_non_finite_keys_stay_with_their_rows(cuda_device, n_win, T, m):
             assert torch.isfinite(got[0][0, s]).all(), f"dq of query {s}"
     keys = [torch.isfinite(r).all(dim=2)[0] for r in ref[1:3]]
     assert all((torch.isfinite(g).all(dim=2)[0] | ~k).all() for g, k in zip(got[1:3], keys))
+
+
+@pytest.mark.parametrize("B,per,S,H,D,n_win,T,m", [(3, 2, 130, 64, 128, 50, 10, 12), (5, 1, 96, 16, 576, 128, 3, 32)])
+def test_groups_of_batches(cuda_device, monkeypatch, B, per, S, H, D, n_win, T, m):
+    # whole batches at a time, the last group shorter: the same sums
+    x = _inputs(B, S, H, D, T, torch.bfloat16, B)
+    whole = _grads(*x, n_win, m)
+    L = _lib.load()
+    group = L.si_hca_attn_bwd_workspace_bytes(per, S, H, D, n_win, T, m, 1 << 40)
+    cap = group + B * S * 64 * 4
+    assert group < L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, T, m, cap) <= cap
+    monkeypatch.setattr(sys.modules[sparse_attn_bwd.__module__], "BWD_WORKSPACE_CAP", cap)
+    assert all(torch.equal(a, b) for a, b in zip(_grads(*x, n_win, m), whole))
+
+
+def test_chunks_of_rows_at_d576(cuda_device, monkeypatch):
+    # two batches of several chunks each, the last chunk's last block short
+    B, S, H, D, n_win, T, m = 2, 1000, 16, 576, 128, 8, 128
+    x = _inputs(B, S, H, D, T, torch.bfloat16, 7)
+    whole = _grads(*x, n_win, m)
+    L = _lib.load()
+    one = L.si_hca_attn_bwd_workspace_bytes(1, S, H, D, n_win, T, m, 1 << 40)
+    cap = one // 2 + (S + T) * D * 4
+    assert 0 < L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, T, m, cap) < one
+    monkeypatch.setattr(sys.modules[sparse_attn_bwd.__module__], "BWD_WORKSPACE_CAP", cap)
+    got = _grads(*x, n_win, m)
+    assert torch.equal(got[0], whole[0]) and torch.equal(got[3], whole[3])
+    _check(got, whole, 2 ** -8, "chunks at D = 576")

@@ -88,3 +88,36 @@ def test_entry_ignores_the_stride_of_a_single_head():
     assert rc == _lib.SI_ERR_INVALID and "workspace" in msg
     rc, msg = _entry(1, 64, 2, 64, 67, 16, 3, 16, hs=1 << 25)
     assert rc == _lib.SI_ERR_UNSUPPORTED and "head stride" in msg
+
+
+def _bytes(*a):
+    if not os.path.exists(LIB_PATH):
+        pytest.skip("libstreamindex.so not built (run __graft_entry__.build())")
+    return _lib.load().si_hca_attn_bwd_workspace_bytes(*a)
+
+
+@pytest.mark.parametrize("B,S,per", [(2, 16384, 1), (4, 8192, 2), (8, 4096, 4), (6, 8192, 3), (5, 8192, 3)])
+def test_plan_takes_whole_batches(B, S, per):
+    # 64 heads, D = 576, window and ratio 128: the default cap holds `per` whole batches in equal groups
+    shape = (S, 64, 576, 128, S // 128, 128)
+    group = _bytes(per, *shape, 1 << 40)
+    assert group <= 2 << 30 < _bytes(B, *shape, 1 << 40)
+    # the plan of a group, and the rest of the batches' dsink terms
+    assert _bytes(B, *shape, 2 << 30) == group + (B - per) * S * 64 * 4
+
+
+def test_plan_parts_are_equal():
+    shape = (1, 20000, 64, 576, 128, 156, 128)
+    whole = _bytes(*shape, 1 << 40)
+    part = _bytes(*shape, whole - 1)
+    acc = 20156 * 576 * 4
+    assert part < 0.6 * whole + acc  # two halves, not all rows but one block and a rest
+
+
+@pytest.mark.parametrize("shape", [(1, 5000, 64, 128, 100, 40, 125), (7, 700, 16, 64, 33, 60, 11), (3, 4097, 130, 576, 128, 32, 128)])
+def test_plan_of_its_own_size_is_itself(shape):
+    whole = _bytes(*shape, 1 << 40)
+    sizes = {_bytes(*shape, int(whole * f)) for f in (0.9, 0.7, 0.5, 0.3, 0.2, 0.1, 0.05)} - {-1}
+    assert len(sizes) > 2
+    for n in sizes:
+        assert _bytes(*shape, n) == n and n < whole
