@@ -66,14 +66,15 @@ __device__ __forceinline__ void hca_item_rows(const HcaBwdArgs& h, int blk, int 
   }
 }
 
-// Index rows [S, 32 wtiles + T] and their used lengths [S], shared by all
-// batches: window column j of query s holds key 32 floor((s-n_win+1)/32) + j
+// Index rows [rows, 32 wtiles + T] of queries s0 .. and their used lengths [rows],
+// shared by all batches: window column j of query s holds key 32 floor((s-n_win+1)/32) + j
 // where that lies in the window, then legal compressed entry i as S + i, else ~key
 // of a key that the query attends to: s, or without a window the first entry
 // (a row without either has length 0).
-__global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t* row_len, int S, int n_win, int T, int m,
-                                                          int wtiles) {
-  const int s = blockIdx.x;
+__global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t* row_len, int s0, int S, int n_win, int T,
+                                                          int m, int wtiles) {
+  const int r = blockIdx.x;
+  const int s = s0 + r;
   const int K = 32 * wtiles + T;
   const int first = s - n_win + 1;
   const int base = (first >> 5) * 32;
@@ -88,9 +89,9 @@ __global__ __launch_bounds__(256) void hca_bwd_idx_kernel(int32_t* idx, int32_t*
       const int i = j - 32 * wtiles;
       v = i < legal ? S + i : masked;
     }
-    idx[static_cast<int64_t>(s) * K + j] = v;
+    idx[static_cast<int64_t>(r) * K + j] = v;
   }
-  if (threadIdx.x == 0) row_len[s] = 32 * wtiles + legal;
+  if (threadIdx.x == 0) row_len[r] = 32 * wtiles + legal;
 }
 
 template <int D>
@@ -472,8 +473,8 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   const int64_t blocks = (rows + RB - 1) / RB;
   p->dsink_rows = take(B * S * 64 * HG * 4);
   p->acc = take(rows < S ? (S + T) * D * 4 : 0);
-  p->idx = take(S * (32 * p->wtiles + T) * 4);
-  p->row_len = take(S * 4);
+  p->idx = take(rows * (32 * p->wtiles + T) * 4);
+  p->row_len = take(rows * 4);
   p->coef = take(nb * rows * HG * p->ntiles * kCoefTile * 2);
   p->part = take(nb * blocks * (p->GW + p->ncg) * kHcaKeys * D * 4);
   p->total = off;
@@ -523,14 +524,9 @@ static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs
   int32_t* idx = reinterpret_cast<int32_t*>(ws + pl.idx);
   int32_t* row_len = reinterpret_cast<int32_t*>(ws + pl.row_len);
   int rc;
-  hipLaunchKernelGGL(hca_bwd_idx_kernel, dim3(static_cast<unsigned>(S)), dim3(256), 0, st, idx, row_len, S, h.n_win, h.T,
-                     h.m, pl.wtiles);
-  if ((rc = check_launch("hca_bwd_idx_kernel"))) return rc;
-  a.idx = idx;
   a.isb = 0;
   a.iss = K;
   a.isk = 1;
-  a.row_len = row_len;
   a.rlsb = 0;
   a.rlss = 1;
   a.K = K;
@@ -552,6 +548,13 @@ static int launch_hca_bwd(AttnBwdArgs a, const HcaPlan& pl, char* ws, HcaBwdArgs
       h.s1 = static_cast<int>(S - s0 < pl.rows ? S : s0 + pl.rows);
       h.first = s0 == 0;
       h.last = h.s1 == S;
+      if (b0 == 0 || pl.rows < S) {  // (whole batches share one chunk's index rows)
+        hipLaunchKernelGGL(hca_bwd_idx_kernel, dim3(static_cast<unsigned>(h.s1 - h.s0)), dim3(256), 0, st, idx, row_len, h.s0,
+                           S, h.n_win, h.T, h.m, pl.wtiles);
+        if ((rc = check_launch("hca_bwd_idx_kernel"))) return rc;
+      }
+      a.idx = idx - s0 * K;  // (indexed by s)
+      a.row_len = row_len - s0;
       a.row0 = b0 * S + s0;
       a.nrows = static_cast<int>(nb * (h.s1 - h.s0));
       const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(a.nrows) * a.HG);

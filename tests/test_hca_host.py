@@ -121,3 +121,10 @@ def test_plan_of_its_own_size_is_itself(shape):
     assert len(sizes) > 2
     for n in sizes:
         assert _bytes(*shape, n) == n and n < whole
+
+
+def test_plan_holds_one_chunk_of_index_rows():
+    # past 215,000 tokens (64 heads, D = 576) the rows of the whole sequence alone fill the default cap
+    S = 262144
+    n = _bytes(1, S, 64, 576, 128, S // 128, 128, 2 << 30)
+    assert 0 < n <= 2 << 30 < S * (160 + S // 128) * 4
