@@ -33,7 +33,7 @@ constexpr int kHcaKeys = 1 << kHcaShift;
 struct HcaBwdArgs {
   int n_win, m, T;
   int wtiles;      // 32-key window tiles of an index row
-  int RB;          // query rows of a block (a multiple of 32)
+  int RB;          // query rows of a block
   int b0;          // first batch of this chunk
   int s0, s1;      // query rows of this chunk (s0 a multiple of RB)
   int GW, ncg;     // window / compressed key groups of a block
@@ -480,18 +480,14 @@ static void hca_plan_for(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_w
   p->total = off;
 }
 
-// The fewest chunks whose plan fits `bytes`; false when none does: all batches, else
-// equal groups of whole batches, else equal parts of one batch's rows (which add up
-// dkv in the workspace).  Equal, because a short last chunk costs what a whole one
-// does on the CUs that it leaves idle.  Row blocks of 64 (fewer partials), smaller
-// where that leaves CUs idle.
-static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, size_t bytes, HcaPlan* p) {
-  for (int RB = 64; RB >= 32; RB /= 2) {
-    hca_plan_for(B, S, H, D, n_win, T, RB, S, B, p);
-    if (RB == 32 || B * ((S + RB - 1) / RB) * (p->GW + p->ncg) >= 512) break;
-  }
+// The plan of row blocks of RB rows with the fewest chunks that fits `bytes`; false
+// when none does: all batches, else equal groups of whole batches, else equal parts
+// of one batch's rows (which add up dkv in the workspace).  Equal, because a short
+// last chunk costs what a whole one does on the CUs that it leaves idle.
+static bool hca_plan_rb(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, int RB, size_t bytes,
+                        HcaPlan* p) {
+  hca_plan_for(B, S, H, D, n_win, T, RB, S, B, p);
   if (p->total <= bytes) return true;
-  const int RB = p->RB;
   // The greatest x below `end` with fits(x) (0: none), then ceil(end / chunks of x).
   auto share = [&](int64_t end, auto fits) {
     int64_t lo = 0, hi = end;
@@ -515,6 +511,27 @@ static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, 
   if (nb > 0) return batches(nb);
   const int64_t n = share((S + RB - 1) / RB, blocks);
   return n > 0 && blocks(n);
+}
+
+// Row blocks of 64 (the fewest partials), smaller where a chunk of them has fewer
+// items than the CUs hold workgroups twice over (two a CU up to D = 256), down to 128
+// stages (of 16 heads of a row) a block: a workgroup of the dkv kernel runs a block's
+// stages one after another.  us a layer step with a floor of 32 rows against this one:
+// 4 x 256 tokens, H = 128, D = 576, n_win = m = 16 612 -> 479 (general backward 508);
+// backward of 64K tokens in chunks of 1,024 (381 MB), D = 576 35.0 -> 27.1 ms (45.7);
+// 1,024 items and not 512 at S = 8,192, H = 64, D = 64, n_win = m = 16 887 -> 783 us (835).
+static bool hca_plan(int64_t B, int64_t S, int64_t H, int64_t D, int64_t n_win, int64_t T, size_t bytes, HcaPlan* p) {
+  bool ok = false;
+  for (int RB = 64; RB >= 8; RB /= 2) {
+    HcaPlan q{};
+    if (hca_plan_rb(B, S, H, D, n_win, T, RB, bytes, &q)) {
+      ok = true;
+      *p = q;
+      if (q.nb * ((q.rows + RB - 1) / RB) * (q.GW + q.ncg) >= (D <= 256 ? 1024 : 512)) break;
+    }
+    if (RB <= 32 && RB * ((H + 15) / 16) <= 128) break;
+  }
+  return ok;
 }
 
 template <int D, bool F16>

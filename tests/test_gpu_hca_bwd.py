@@ -69,6 +69,10 @@ def _check(got, ref, eps, label):
     (1, 90, 64, 128, 16, 50, 4, torch.bfloat16),      # entries past the last legal one
     (1, 1, 64, 576, 128, 0, 128, torch.bfloat16),
     (1, 4000, 16, 64, 128, 31, 128, torch.bfloat16),
+    (1, 8200, 16, 512, 128, 64, 128, torch.bfloat16),  # blocks of 64 rows, the last one of 8
+    (2, 6150, 4, 32, 128, 1000, 6, torch.float16),     # the same, one batch at a time
+    (1, 330, 128, 576, 128, 2, 128, torch.bfloat16),   # blocks of 16
+    (1, 77, 300, 64, 40, 9, 8, torch.float16),         # blocks of 8
 ])
 def test_matches_general_backward(cuda_device, B, S, H, D, n_win, T, m, dt):
     assert _lib.load().si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, T, m, 1 << 31) > 0
@@ -209,3 +213,18 @@ def test_chunks_of_rows_at_d576(cuda_device, monkeypatch):
     got = _grads(*x, n_win, m)
     assert torch.equal(got[0], whole[0]) and torch.equal(got[3], whole[3])
     _check(got, whole, 2 ** -8, "chunks at D = 576")
+
+
+def test_chunks_of_64_row_blocks(cuda_device, monkeypatch):
+    # two parts of a batch, blocks of 64 rows in both
+    B, S, H, D, n_win, T, m = 1, 8400, 4, 512, 128, 640, 13
+    x = _inputs(B, S, H, D, T, torch.bfloat16, 11)
+    whole = _grads(*x, n_win, m)
+    L = _lib.load()
+    need = L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, T, m, 1 << 40)
+    got = L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, T, m, need - 1)
+    assert 0 < got < 0.6 * need
+    monkeypatch.setattr(sys.modules[sparse_attn_bwd.__module__], "BWD_WORKSPACE_CAP", need - 1)
+    part = _grads(*x, n_win, m)
+    assert torch.equal(part[0], whole[0]) and torch.equal(part[3], whole[3])
+    _check(part, whole, 2 ** -8, "parts of 64-row blocks")

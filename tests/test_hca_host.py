@@ -128,3 +128,37 @@ def test_plan_holds_one_chunk_of_index_rows():
     S = 262144
     n = _bytes(1, S, 64, 576, 128, S // 128, 128, 2 << 30)
     assert 0 < n <= 2 << 30 < S * (160 + S // 128) * 4
+
+
+def _plan_bytes(B, S, H, D, n_win, T, RB, rows=None):
+    """Workspace of all batches in row blocks of RB, or of one batch in parts of `rows` rows."""
+    nb, rows = (B, S) if rows is None else (1, rows)
+    HG, wt = (H + 63) // 64, (n_win + 62) // 32 if n_win else 0
+    GW, ncg = (RB + n_win - 2) // 128 + 2 if n_win else 0, (T + 127) // 128
+    sizes = (B * S * 64 * HG * 4, (S + T) * D * 4 if rows < S else 0, rows * (32 * wt + T) * 4, rows * 4,
+             nb * rows * HG * (wt + (T + 31) // 32) * 8192, nb * ((rows + RB - 1) // RB) * (GW + ncg) * 128 * D * 4)
+    return sum((n + 255) // 256 * 256 for n in sizes)
+
+
+@pytest.mark.parametrize("B,S,H,D,n_win,T,RB", [
+    (1, 16384, 64, 576, 128, 128, 64),
+    (1, 8200, 16, 512, 128, 64, 64),
+    (1, 4096, 64, 576, 128, 32, 32),
+    (1, 8192, 64, 256, 128, 64, 32),    # two workgroups a CU up to D = 256
+    (2, 9000, 16, 64, 128, 1000, 64),
+    (1, 300, 16, 64, 128, 2, 32),       # few stages a block: 32 rows at least
+    (1, 300, 64, 576, 128, 2, 32),
+    (4, 256, 128, 576, 16, 16, 16),
+    (1, 300, 256, 64, 128, 2, 8),
+    (1, 300, 600, 64, 128, 2, 8),
+])
+def test_row_blocks(B, S, H, D, n_win, T, RB):
+    assert _bytes(B, S, H, D, n_win, T, 128, 1 << 40) == _plan_bytes(B, S, H, D, n_win, T, RB)
+
+
+def test_row_blocks_of_parts():
+    # 132 blocks of 64 rows in two parts; 16,384 tokens in parts of 1,024 rows take blocks of 32
+    shape = (1, 8400, 4, 512, 128, 640)
+    assert _bytes(*shape, 13, _plan_bytes(*shape, 64) - 1) == _plan_bytes(*shape, 64, 66 * 64)
+    shape = (1, 16384, 64, 576, 128, 128)
+    assert _bytes(*shape, 128, _plan_bytes(*shape, 32, 1024)) == _plan_bytes(*shape, 32, 1024)
