@@ -190,7 +190,9 @@ int si_sparse_attn_fwd_kv2(const void* q, const int64_t* q_strides, const void* 
  * split each row's columns over several workgroups and combine their fp32
  * partial outputs.  si_sparse_attn_fwd_scratch_bytes says how much such a call
  * needs, 0 for calls that take none; with a scratch that is NULL or smaller
- * the call runs unsplit.  No counterpart in the reference.
+ * the call runs unsplit.  Split results differ from unsplit ones by rounding (P
+ * relative to each split's own maximum); either repeats bit for bit.  No
+ * counterpart in the reference.
  */
 int64_t si_sparse_attn_fwd_scratch_bytes(int64_t B, int64_t S, int64_t H, int64_t D, int64_t K);
 int si_sparse_attn_fwd_scratch(const void* q, const int64_t* q_strides, const void* kv, const int64_t* kv_strides,
@@ -244,7 +246,7 @@ int si_hca_topk_idxs(int64_t B, int64_t S, int64_t n_win, int64_t n_compressed, 
                      int64_t idx_offset, int32_t* out_idx, const int64_t* out_strides, void* stream);
 
 /*
- * Used columns of CSA / HCA index rows, out[s] = n_win + min(cap, (s+1)/m) for
+ * Used columns of CSA / HCA index rows, int32 sizes, out[s] = n_win + min(cap, (s+1)/m) for
  * s < S (cap: picks per row), the row lengths the attention entries take.
  */
 int si_row_len(int64_t S, int64_t n_win, int64_t cap, int64_t m, int32_t* out, void* stream);

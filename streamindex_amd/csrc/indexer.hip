@@ -19,6 +19,7 @@ int g_topk_kernel_mode = 0;
 // and past the line 1,536 x 2,048  79 -> 85, 2,048 x 32,000  818 -> 916: there
 // the one-wave-per-row kernel fills the chip and saves the scores' round trip.
 constexpr int64_t kFewMaxGroups = 256;
+// (a bound on what a call allocates; 256 rows x 262,144 keys are just past it)
 constexpr int64_t kFewMaxScratch = int64_t(256) << 20;
 
 // Kernel and selection capacity for a top-k shape.  A compaction keeps

@@ -770,7 +770,10 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(SparseAttnArgs
 // tiles while other CUs idle; the second launch and the fp32 partial outputs
 // take back 7 us and 0.6 us a MB, so rows split where that saves a quarter of
 // the estimate: 1 row x K = 2,048 78 -> 27 us, 16 x 2,048 78 -> 31, 16 x 1,024
-// 44 -> 28, 64 x 2,048 79 -> 47; 16 x 512 (25 us) stays whole.
+// 44 -> 28, 64 x 2,048 79 -> 47; 16 x 512 (25 us) stays whole.  The same estimate
+// scaled by D (H = 64): at D = 256 1 x 1,024 32 -> 22, 64 x 2,048 60 -> 34, 16 x 1,024
+// (33) whole; at D = 128 1 x 1,024 24 -> 22, 64 x 2,048 45 -> 26; at D = 64 16 x 2,048
+// 38 -> 21, 1 x 1,024 20.7 -> 21.2 at the line itself.
 struct AttnPlan {
   int mode, splits, span;
   int64_t bytes;  // scratch of the split rows
