@@ -293,7 +293,7 @@ __global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(Attn
       }
       attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
     }
-    float z = 0.f;  // NaN where a sum is not finite
+    f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};  // NaN where a sum is not finite
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
 #pragma unroll
@@ -302,11 +302,11 @@ __global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(Attn
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) z = __builtin_fmaf(acc[m][nb][c], 0.f, z);
+          for (int c = 0; c < 4; ++c) z[c] = __builtin_fmaf(acc[m][nb][c], 0.f, z[c]);
       }
     }
     // (before the stores: an LDS read waits for the memory operations in flight)
-    const bool bad = __builtin_amdgcn_ballot_w64(z != 0.f) != 0;
+    const bool bad = __builtin_amdgcn_ballot_w64((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0;
     if (lane == 0) nonfinite_lds[wave] = bad ? 1 : 0;
     attn_tile_barrier();
     int any = 0;
