@@ -408,8 +408,8 @@ __global__ __launch_bounds__(kFewThreads) void few_select_kernel(FewSelectArgs a
     int bin[ES], slot[ES];
 #pragma unroll
     for (int j = 0; j < ES; ++j) {
-      bin[j] = static_cast<int>((top - ord_to_f32(key_hi(v[j]))) * scale);
-      bin[j] = bin[j] < BINS - 1 ? bin[j] : BINS - 1;
+      // (an empty slot's score is NaN: the minimum takes the bound)
+      bin[j] = static_cast<int>(__builtin_fminf((top - ord_to_f32(key_hi(v[j]))) * scale, static_cast<float>(BINS - 1)));
       slot[j] = v[j] != 0ull ? atomicAdd(&hist[bin[j]], 1) : 0;
     }
     __syncthreads();
