@@ -97,15 +97,34 @@ class _HcaAttnFunc(torch.autograd.Function):
         return dq, dkv[:, :n1], dkv[:, n1:], dsink, None, None, None
 
 
+def _general_is_faster(rows: int, H: int, D: int, n_win: int, picks: float) -> bool:
+    """Whether the general backward is faster than the aligned one for ``rows`` queries (batches included) with a window
+    of ``n_win`` and ``picks`` compressed entries each on average.
+
+    A 128-key group that a query meets costs the aligned path the same whatever it holds; a pair costs the general one a
+    16-bit row, little at D <= 128.  So the keys per group decide, once the launches (twice as many in the general
+    path) no longer count, and not with up to 32 heads, where the general path works in steps of 64.  us a step,
+    general against aligned, m = 128 unless given:
+      D = 64, 20,000 queries, H = 64: n_win = 16 (42 keys a group) 950, 1,262; 64 (55) 1,152, 1,347; 128 (66) 1,426, 1,396;
+        n_win = 0, m = 32 (71) 859, 852; 4,000 queries, n_win = m = 64 480, 367; H = 32, 16,384 queries, m = 64 1,321, 915
+      D = 128, 20,000 queries, H = 64: n_win = 16 (42) 1,480, 1,644; 64 (55) 1,785, 1,739; n_win = 128,
+        m = 500 (52) 1,589, 1,716; H = 128 10,000 queries, n_win = 64 2,069, 1,442; nothing at D = 256."""
+    least = 64 if D <= 64 else 53 if D == 128 and H <= 64 else 0
+    groups = (1 + (n_win - 1) / 128 if n_win else 0) + (picks / 128 + 0.5 if picks else 0)
+    return H > 32 and rows * ((H + 63) // 64) > 8192 and n_win + picks < least * groups
+
+
 def _hca_attn_bwd(q, kv, attn_sink, o, lse, do, n_compressed, softmax_scale, n_win, m_prime):
     """``(dq, dkv, dsink)`` for ``kv = [kv ; kv_compressed]``, by ``si_hca_attn_bwd`` where it serves the shape (one kv row
-    per query) and its workspace fits the backward's cap, else by the general backward over the index rows."""
+    per query), is the faster one and its workspace fits the backward's cap, else by the general backward over the index
+    rows."""
     B, S, H, D = q.shape
     N_kv = kv.shape[1]
     L = _lib.load()
     with _lib.on_device(q.device):
         ws = None
-        if N_kv == S + n_compressed:
+        picks = min(n_compressed, S // m_prime) / 2
+        if N_kv == S + n_compressed and not _general_is_faster(B * S, H, D, min(n_win, S), picks):
             ws = _bwd_workspace(
                 lambda cap: L.si_hca_attn_bwd_workspace_bytes(B, S, H, D, n_win, n_compressed, m_prime, cap), None, q.device)
         if ws is None:

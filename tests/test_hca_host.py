@@ -162,3 +162,15 @@ def test_row_blocks_of_parts():
     assert _bytes(*shape, 13, _plan_bytes(*shape, 64) - 1) == _plan_bytes(*shape, 64, 66 * 64)
     shape = (1, 16384, 64, 576, 128, 128)
     assert _bytes(*shape, 128, _plan_bytes(*shape, 32, 1024)) == _plan_bytes(*shape, 32, 1024)
+
+
+@pytest.mark.parametrize("rows,H,D,n_win,picks,general", [
+    (20000, 64, 64, 16, 78, True), (20000, 64, 64, 64, 78, True), (20000, 64, 64, 128, 78, False),
+    (20000, 64, 64, 0, 78, False), (20000, 64, 64, 1, 0, True), (20000, 64, 32, 0, 0, False),
+    (8192, 64, 64, 16, 78, False), (8193, 64, 64, 16, 78, True), (4097, 128, 32, 16, 20, True),
+    (20000, 32, 64, 16, 78, False), (20000, 33, 64, 16, 78, True),
+    (20000, 64, 128, 16, 78, True), (20000, 64, 128, 64, 78, False), (20000, 65, 128, 16, 78, False),
+    (20000, 64, 256, 16, 78, False), (60000, 64, 576, 1, 20, False),
+])
+def test_few_keys_a_group_take_the_general_backward(rows, H, D, n_win, picks, general):
+    assert hca._general_is_faster(rows, H, D, n_win, picks) == general
