@@ -14,7 +14,8 @@
 //      every tile (8 KiB each) in its register layout.
 //   3. hca_bwd_dkv_kernel: per (128 keys, RB query rows) the sum over the rows'
 //      heads of dS q + P dO, fp32, to a partial buffer.  Sums that are not finite
-//      are taken again row by row, with only the keys each row attends to.
+//      are taken again with each stage apart, for the keys its row attends to only
+//      (S = 16,384, D = 576: a step 4.2 ms, 5.1 with one infinity, 9.0 with NaN in every row).
 //   4. hca_bwd_reduce_kernel: each key's partials in block order.
 // Every sum has a fixed order, so repeated calls are bit-identical.
 //
@@ -227,72 +228,122 @@ __global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(Attn
   const uint32_t qd0 = lds_addr(qd_lds) + (g >> 1) * HS::PART + kh * HS::QROW + 8 * (i16 & 3) + blk_lo * 32;
   const uint32_t cf0 = lds_addr(coef_lds) + (g < 2 ? HS::CW4 : 0) + (i16 & 3) * HS::CG + kh * 16;
 
+  // Whether query s attends to this lane's key of key block nb.
+  auto attends = [&](int s, int nb) {
+    const int key = kt * 32 + nb * 16 + i16;
+    return window ? key <= s && key > s - h.n_win : key < h.T && static_cast<int64_t>(h.m) * (key + 1) <= s + 1;
+  };
+
   // The stages with NB dimension blocks (a compile-time count: LDS reads in
   // flight must not cross control flow, where their registers could be copied
   // before the data lands).
   auto stages = [&](auto NBC) {
     constexpr int NB = decltype(NBC)::value;
     f32x4 acc[NB > 0 ? NB : 1][8];
+    // The sums over all stages.  APART: each stage's part is formed apart and added for
+    // the keys that its row attends to only.
+    auto sum_stages = [&](auto APARTC) {
+      constexpr bool APART = decltype(APARTC)::value;
 #pragma unroll
-    for (int m = 0; m < NB; ++m)
+      for (int m = 0; m < NB; ++m)
 #pragma unroll
-      for (int nb = 0; nb < 8; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    Stage cur{r0, 0};
-    copy_stage(cur, 0);
-    load_coef(cur);
-    int buf = 0;
-    for (; cur.s < r1; buf ^= 1) {
-      __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));  // this stage's copies and coefficients landed (issued a stage ago)
-      *reinterpret_cast<u32x4*>(cst) = cf;
-      attn_tile_barrier();
-      // (the other buffer was last read in the previous stage, which every wave has left)
-      cur = next(cur);
-      if (cur.s < r1) {
-        copy_stage(cur, buf ^ 1);
-        load_coef(cur);
-      }
-      if constexpr (NB > 0) {
-        // Key blocks nb: 16 (nb & 1) of tile nb >> 1.
-        v4i16 blo[8], bhi[8];
-        attn_static_for<0, 8>([&](auto NC) {
-          constexpr int nb = decltype(NC)::value;
-          constexpr int off = (nb >> 1) * 2 * HS::CW4 + 8 * (nb & 1);
-          blo[nb] = tr_read<off>(cf0);
-          bhi[nb] = tr_read<off + 64>(cf0);
-        });
-        const uint32_t qa = qd0 + buf * HS::BUF;
-        v4i16 alo[2], ahi[2];
-        auto a_read = [&](auto JC) {
-          constexpr int m = decltype(JC)::value;
-          alo[m & 1] = tr_read<m * 32>(qa);
-          ahi[m & 1] = tr_read<m * 32 + 4 * HS::QROW>(qa);
-        };
-        a_read(std::integral_constant<int, 0>{});
-        lds_wait_n<2>();
-        bf16x8 bfr[8];
-#pragma unroll
-        for (int nb = 0; nb < 8; ++nb) {
-          reg_tie(blo[nb]);
-          reg_tie(bhi[nb]);
-          bfr[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[nb], bhi[nb], 0, 1, 2, 3, 4, 5, 6, 7));
+        for (int nb = 0; nb < 8; ++nb) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      Stage cur{r0, 0};
+      copy_stage(cur, 0);
+      load_coef(cur);
+      int buf = 0;
+      for (; cur.s < r1; buf ^= 1) {
+        const int s = cur.s;
+        __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));  // this stage's copies and coefficients landed (issued a stage ago)
+        *reinterpret_cast<u32x4*>(cst) = cf;
+        attn_tile_barrier();
+        // (the other buffer was last read in the previous stage, which every wave has left)
+        cur = next(cur);
+        if (cur.s < r1) {
+          copy_stage(cur, buf ^ 1);
+          load_coef(cur);
         }
-        attn_static_for<0, NB>([&](auto JC) {
-          constexpr int m = decltype(JC)::value;
-          if constexpr (m + 1 < NB) {
-            a_read(std::integral_constant<int, m + 1>{});
-            lds_wait_n<2>();
-          } else {
-            lds_wait_n<0>();
-          }
-          reg_tie(alo[m & 1]);
-          reg_tie(ahi[m & 1]);
-          const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo[m & 1], ahi[m & 1], 0, 1, 2, 3, 4, 5, 6, 7));
+        if constexpr (NB > 0 && !APART) {
+          // Key blocks nb: 16 (nb & 1) of tile nb >> 1.
+          v4i16 blo[8], bhi[8];
+          attn_static_for<0, 8>([&](auto NC) {
+            constexpr int nb = decltype(NC)::value;
+            constexpr int off = (nb >> 1) * 2 * HS::CW4 + 8 * (nb & 1);
+            blo[nb] = tr_read<off>(cf0);
+            bhi[nb] = tr_read<off + 64>(cf0);
+          });
+          const uint32_t qa = qd0 + buf * HS::BUF;
+          v4i16 alo[2], ahi[2];
+          auto a_read = [&](auto JC) {
+            constexpr int m = decltype(JC)::value;
+            alo[m & 1] = tr_read<m * 32>(qa);
+            ahi[m & 1] = tr_read<m * 32 + 4 * HS::QROW>(qa);
+          };
+          a_read(std::integral_constant<int, 0>{});
+          lds_wait_n<2>();
+          bf16x8 bfr[8];
 #pragma unroll
-          for (int nb = 0; nb < 8; ++nb) acc[m][nb] = mfma16x16x32<F16>(af, bfr[nb], acc[m][nb]);
-        });
+          for (int nb = 0; nb < 8; ++nb) {
+            reg_tie(blo[nb]);
+            reg_tie(bhi[nb]);
+            bfr[nb] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[nb], bhi[nb], 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+          attn_static_for<0, NB>([&](auto JC) {
+            constexpr int m = decltype(JC)::value;
+            if constexpr (m + 1 < NB) {
+              a_read(std::integral_constant<int, m + 1>{});
+              lds_wait_n<2>();
+            } else {
+              lds_wait_n<0>();
+            }
+            reg_tie(alo[m & 1]);
+            reg_tie(ahi[m & 1]);
+            const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo[m & 1], ahi[m & 1], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) acc[m][nb] = mfma16x16x32<F16>(af, bfr[nb], acc[m][nb]);
+          });
+        }
+        if constexpr (NB > 0 && APART) {
+          // (two key blocks at a time, so that this takes no more registers than the above)
+          const uint32_t qa = qd0 + buf * HS::BUF;
+          attn_static_for<0, NB>([&](auto JC) {
+            constexpr int m = decltype(JC)::value;
+            attn_static_for<0, 4>([&](auto NC) {
+              constexpr int n = decltype(NC)::value;
+              v4i16 alo = tr_read<m * 32>(qa);
+              v4i16 ahi = tr_read<m * 32 + 4 * HS::QROW>(qa);
+              v4i16 xlo = tr_read<n * 2 * HS::CW4>(cf0);
+              v4i16 xhi = tr_read<n * 2 * HS::CW4 + 64>(cf0);
+              v4i16 ylo = tr_read<n * 2 * HS::CW4 + 8>(cf0);
+              v4i16 yhi = tr_read<n * 2 * HS::CW4 + 8 + 64>(cf0);
+              lds_wait_n<0>();
+              reg_tie(alo);
+              reg_tie(ahi);
+              reg_tie(xlo);
+              reg_tie(xhi);
+              reg_tie(ylo);
+              reg_tie(yhi);
+              const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo, ahi, 0, 1, 2, 3, 4, 5, 6, 7));
+              const bf16x8 xf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(xlo, xhi, 0, 1, 2, 3, 4, 5, 6, 7));
+              const bf16x8 yf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(ylo, yhi, 0, 1, 2, 3, 4, 5, 6, 7));
+              f32x4 x = mfma16x16x32<F16>(af, xf, f32x4{0.f, 0.f, 0.f, 0.f});
+              f32x4 y = mfma16x16x32<F16>(af, yf, f32x4{0.f, 0.f, 0.f, 0.f});
+              mfma_result_fence(x, y);
+              const bool bx = attends(s, 2 * n), by = attends(s, 2 * n + 1);
+#pragma unroll
+              for (int c = 0; c < 4; ++c) {
+                acc[m][2 * n][c] = bx ? acc[m][2 * n][c] + x[c] : acc[m][2 * n][c];
+                acc[m][2 * n + 1][c] = by ? acc[m][2 * n + 1][c] + y[c] : acc[m][2 * n + 1][c];
+              }
+              reg_tie(acc[m][2 * n]);  // (added here, not after later parts)
+              reg_tie(acc[m][2 * n + 1]);
+            });
+          });
+        }
+        attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
       }
-      attn_tile_barrier();  // every wave is done with this stage's coefficients and buffer
-    }
+    };
+    sum_stages(std::false_type{});
     f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};  // NaN where a sum is not finite
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
@@ -305,13 +356,19 @@ __global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(Attn
           for (int c = 0; c < 4; ++c) z[c] = __builtin_fmaf(acc[m][nb][c], 0.f, z[c]);
       }
     }
-    // (before the stores: an LDS read waits for the memory operations in flight)
+    // (before the stores: an LDS read waits for the memory operations in flight.  The
+    // barrier also ends every wave's use of the buffers.)
     const bool bad = __builtin_amdgcn_ballot_w64((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0;
     if (lane == 0) nonfinite_lds[wave] = bad ? 1 : 0;
     attn_tile_barrier();
     int any = 0;
 #pragma unroll
     for (int w = 0; w < HS::NW; ++w) any |= nonfinite_lds[w];
+    if (__builtin_amdgcn_readfirstlane(any) != 0) {
+      // The coefficients of the keys that a row does not attend to are 0, and 0
+      // times an infinity or NaN of the row's Q or dO is NaN.
+      sum_stages(std::true_type{});
+    }
     // lane (key 16 nb + i16 of the group, g) holds dimensions 16 mbi + 4 g + 0..3
     float* out = h.part + static_cast<int64_t>(item) * kHcaKeys * D;
 #pragma unroll
@@ -320,78 +377,6 @@ __global__ __launch_bounds__(512, D <= 256 ? 4 : 2) void hca_bwd_dkv_kernel(Attn
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb)
           *reinterpret_cast<f32x4*>(out + (nb * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = acc[m][nb];
-      }
-    }
-    if (__builtin_amdgcn_readfirstlane(any) != 0) {
-      // The coefficients of the keys that a row does not attend to are 0, and 0
-      // times an infinity or NaN of the row's Q or dO is NaN.  So: one dimension
-      // block and KH of the group's 16-key blocks at a time (no more registers than
-      // the loop above takes), a row's sum over its heads apart, added for the keys
-      // that the row attends to.  (8 / KH MBW passes over the stages instead of one.)
-      constexpr int KH = 4;
-      for (int pass = 0; pass < 8 / KH * MBW; ++pass) {
-        const int m = pass / (8 / KH), n0 = pass % (8 / KH) * KH;
-        const bool has = m < NB;
-        const uint32_t ca = cf0 + n0 * HS::CW4;
-        f32x4 row[KH], tot[KH];
-#pragma unroll
-        for (int nb = 0; nb < KH; ++nb) row[nb] = tot[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        cur = Stage{r0, 0};
-        copy_stage(cur, 0);
-        load_coef(cur);
-        for (buf = 0; cur.s < r1; buf ^= 1) {
-          __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));
-          *reinterpret_cast<u32x4*>(cst) = cf;
-          attn_tile_barrier();
-          const Stage at = cur;
-          cur = next(cur);
-          if (cur.s < r1) {
-            copy_stage(cur, buf ^ 1);
-            load_coef(cur);
-          }
-          if (has) {
-            v4i16 blo[KH], bhi[KH];
-            attn_static_for<0, KH>([&](auto NC) {
-              constexpr int nb = decltype(NC)::value;
-              constexpr int off = (nb >> 1) * 2 * HS::CW4 + 8 * (nb & 1);
-              blo[nb] = tr_read<off>(ca);
-              bhi[nb] = tr_read<off + 64>(ca);
-            });
-            const uint32_t qa = qd0 + buf * HS::BUF + m * 32;
-            v4i16 alo = tr_read<0>(qa);
-            v4i16 ahi = tr_read<4 * HS::QROW>(qa);
-            lds_wait_n<0>();
-            reg_tie(alo);
-            reg_tie(ahi);
-            const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(alo, ahi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int nb = 0; nb < KH; ++nb) {
-              reg_tie(blo[nb]);
-              reg_tie(bhi[nb]);
-              const bf16x8 bf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(blo[nb], bhi[nb], 0, 1, 2, 3, 4, 5, 6, 7));
-              if (at.part == 0) row[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-              row[nb] = mfma16x16x32<F16>(af, bf, row[nb]);
-            }
-            if (at.part == nq - 1) {
-#pragma unroll
-              for (int nb = 0; nb < KH; nb += 2) mfma_result_fence(row[nb], row[nb + 1]);
-#pragma unroll
-              for (int nb = 0; nb < KH; ++nb) {
-                const int key = kt * 32 + (n0 + nb) * 16 + i16;
-                const bool attends = window ? key <= at.s && key > at.s - h.n_win
-                                            : key < h.T && static_cast<int64_t>(h.m) * (key + 1) <= at.s + 1;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) tot[nb][c] = attends ? tot[nb][c] + row[nb][c] : tot[nb][c];
-              }
-            }
-          }
-          attn_tile_barrier();
-        }
-        if (has && blk_lo + m < HS::MBT) {
-#pragma unroll
-          for (int nb = 0; nb < KH; ++nb)
-            *reinterpret_cast<f32x4*>(out + ((n0 + nb) * 16 + i16) * D + (blk_lo + m) * 16 + 4 * g) = tot[nb];
-        }
       }
     }
   };
